@@ -8,21 +8,23 @@
 //    v_mfma_f32_32x32x2f32 tiles (FP32 inputs, FP32 accumulate). The matrix
 //    core sums k-slices in its own order, so results match the reference's
 //    ascending-k FMA chain within FP32 rounding (tolerance).
-//  - chain2_kernel (k a multiple of 16) / chain_kernel (any shape): SIMT
-//    register tiles in which every output is one FMA chain over ascending k
-//    from +0.0: bitwise the reference's FP32 panels.
+//  - chain_mfma_kernel (gemm_chain.hip: k a multiple of 64, no exception
+//    columns) on the FP32 matrix cores, and for the other shapes
+//    chain2_kernel (k a multiple of 16) / chain_kernel (any shape), SIMT
+//    register tiles: every output is one FMA chain over ascending k from +0.0,
+//    bitwise the reference's FP32 panels.
 // INT16 / INT8 codes are read as codes by every kernel and turned into
 // fl(code * scale) in registers (in dma_kernel as the B fragments are read,
 // in the others on the way into LDS); no FP32 copy of a code matrix is ever
 // written to memory.
 //
-// Roofline: FP32 matrix cores (157.3 TFLOP/s) for mfma_kernel; the FP32
-// vector peak (157.3 TFLOP/s: gfx950 issues even non-packed FMAs faster than
-// 16 lanes per clock, measured 114 TFLOP/s for a register-only FMA loop) for
-// the chain kernels. FLOPs = 2*m*k*n.
+// Roofline: FP32 matrix cores (157.3 TFLOP/s) for the matrix-core kernels; the
+// FP32 vector peak (157.3 TFLOP/s: gfx950 issues even non-packed FMAs faster
+// than 16 lanes per clock, measured 114 TFLOP/s for a register-only FMA loop)
+// for the SIMT chain kernels. FLOPs = 2*m*k*n.
 #include <type_traits>
 
-#include "focr_internal.hpp"
+#include "gemm_f32.hpp"
 
 namespace focr {
 namespace {
@@ -58,20 +60,6 @@ __device__ __forceinline__ float weight_at(const T *__restrict__ codes, const fl
   return w;
 }
 
-struct GemmArgs {
-  const float *x;
-  const float *row_scale;
-  const void *codes;
-  const float *scales;
-  const int16_t *exc_index;
-  const int32_t *exc_cols;
-  const float *exc_vals;
-  int n_exc;
-  int m, n, k, group, groups;
-  float *out;
-  int row0;  // dma_kernel: first output row of the launch's tiles (0 for the other kernels)
-};
-
 // Stages A'[m0.., k0..k0+32) and W[n0.., k0..k0+32) into LDS as [row][k].
 template <typename T, int ROWS>
 __device__ __forceinline__ void stage_tiles(const GemmArgs &a, int m0, int n0, int k0, float (*as)[kPitch],
@@ -94,21 +82,6 @@ __device__ __forceinline__ void stage_tiles(const GemmArgs &a, int m0, int n0, i
     if (row < a.n && col < a.k)
       w = weight_at<T>(codes, a.scales, a.exc_index, a.exc_vals, a.n_exc, a.k, a.group, a.groups, row, col);
     bs[r][c] = w;
-  }
-}
-
-// Writes one output value through the epilogue. For GLU, `partner` is the
-// value of the neighbouring column (col ^ 1), fetched by the caller.
-template <int EPI>
-__device__ __forceinline__ void emit(const GemmArgs &a, int row, int col, float v, float partner) {
-  if (row >= a.m || col >= a.n) return;
-  if constexpr (EPI == FOCR_EPI_GLU) {
-    if ((col & 1) == 0) a.out[static_cast<size_t>(row) * (a.n / 2) + col / 2] = squared_relu_glu(v, partner);
-  } else if constexpr (EPI == FOCR_EPI_ADD) {
-    float *dst = a.out + static_cast<size_t>(row) * a.n + col;
-    *dst = *dst + v;
-  } else {
-    a.out[static_cast<size_t>(row) * a.n + col] = v;
   }
 }
 
@@ -319,23 +292,9 @@ __global__ __launch_bounds__(256) void mfma_kernel(GemmArgs a) {
 //    The codes of exception columns are zero (upload refuses others), so each
 //    exception adds a'[r][col_e] * value[c][e] to the sums before the
 //    epilogue; the matrix cores sum in their own order anyway.
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void global_void;
-
 constexpr int kDmaBK = 16;
 
 __device__ __forceinline__ int dma_swizzle(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
-
-// s_waitcnt immediate for vmcnt(n) (n < 64) and lgkmcnt(0), expcnt not waited.
-constexpr int wait_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0070; }
-
-// Compiler-only ordering around the plain workgroup barrier: the waits are
-// explicit (a __syncthreads fence would wait for every copy in flight).
-__device__ __forceinline__ void plain_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 template <typename T, int EPI, int BN, int BM = 128>
 __global__ __launch_bounds__(256) void dma_kernel(GemmArgs a) {
@@ -808,6 +767,8 @@ void launch_one(bool chain, const GemmArgs &a, hipStream_t stream) {
     if (a.k % kC2K == 0 && aligned && (std::is_same<T, float>::value || a.group % 8 == 0)) {
       // 128 x 128 tiles where they give at least two per compute unit,
       // 64 x 64 ones otherwise (n = 768 at 6,544 rows: WO 0.264 -> 0.195 ms).
+      // Only exception columns, k not a multiple of 64 and groups of 32
+      // reach these.
       const long big = static_cast<long>((a.m + 127) / 128) * ((a.n + 127) / 128);
       if (big >= 512)
         hipLaunchKernelGGL((chain2_kernel<T, EPI, 128, 128>), dim3((a.m + 127) / 128, (a.n + 127) / 128), dim3(256), 0,
@@ -1077,23 +1038,6 @@ union PairFrag {
 // 16 distinct bank groups. Step st reads stage st's fragments while the
 // products of stage st - 1 run. Rows and columns are padded to 128 with zeros
 // in the planes; outputs past m or n are not written.
-// Tile order: workgroups are dealt to the 8 XCDs round robin (block b runs on
-// XCD b % 8); block b takes tile t = (b % 8) * per + b / 8, so each XCD walks
-// a contiguous run of tiles, in panels of kSplitPanel row tiles (column tiles
-// in order, rows fastest): the workgroups an XCD holds at once share a few A
-// row tiles and B column tiles in its own L2.
-constexpr int kSplitPanel = 4;
-__device__ __forceinline__ void split_tile(int b, int row_tiles, int col_tiles, int &rt, int &ct) {
-  const int total = row_tiles * col_tiles;
-  const int per = total / 8;
-  const int t = b < 8 * per ? (b % 8) * per + b / 8 : b;
-  const int panel = t / (kSplitPanel * col_tiles);
-  const int rem = t - panel * kSplitPanel * col_tiles;
-  const int rows = row_tiles - panel * kSplitPanel < kSplitPanel ? row_tiles - panel * kSplitPanel : kSplitPanel;
-  ct = rem / rows;
-  rt = panel * kSplitPanel + rem % rows;
-}
-
 template <int EPI, int BM>
 __global__ __launch_bounds__(256) void split_kernel(GemmArgs a, const uint16_t *__restrict__ ap,
                                                     const uint16_t *__restrict__ bp, const int *__restrict__ aexp,
@@ -1115,7 +1059,7 @@ __global__ __launch_bounds__(256) void split_kernel(GemmArgs a, const uint16_t *
   const int wm = wave >> 1, wn = wave & 1;
   if (tid == 0) tile_any = 0;  // the main loop's barriers order it before the epilogue's writes
   int rt, ct;
-  split_tile(blockIdx.x, row_tiles, col_tiles, rt, ct);
+  xcd_tile(blockIdx.x, row_tiles, col_tiles, rt, ct);
   const int m0 = a.row0 + rt * BM, n0 = ct * kSplitBN;
   const int h = lane >> 5, l32 = lane & 31;
   // Copy t of operand o fills slots q = 64 (wave + 4 t) + lane: plane q / S,
@@ -1368,6 +1312,10 @@ int launch_f32_common(bool chain, Ctx *ctx, const Linear *lin, const float *x, s
   // in place) in registers from the uploaded matrix; no FP32 copy of the
   // weights is written.
   const GemmArgs a = make_args(lin, x, rows, row_scale, out);
+  if (chain && launch_chain_mfma(a, lin->bits, epilogue, ctx->stream)) {
+    FOCR_HIP_CHECK(hipGetLastError());
+    return FOCR_OK;
+  }
   if (lin->bits == 8)
     launch_epi<int8_t>(chain, epilogue, a, ctx->stream);
   else if (lin->bits == 16)
