@@ -1217,6 +1217,117 @@ __global__ __launch_bounds__(256) void split_kernel(GemmArgs a, const uint16_t *
   }
 }
 
+// Small grids: (32 IB) x (32 JB) outputs per workgroup of WK waves, each wave
+// all of them over every WK-th 16-k stage, its fragments loaded straight into
+// registers D stages ahead (a stage of 32 consecutive rows of a plane is one
+// contiguous 1 KB run in fragment order), the waves' sums added through LDS in
+// wave order. Flagged outputs are recomputed by the FP32 chain.
+// Bound: latency. split_kernel's tiles leave a small grid with a few
+// workgroups that each walk all of k, a barrier and an exposed load per 16-k
+// stage (about 0.3 us a stage); here a wave walks 1 / WK of it, without
+// barriers. m = 144, us, this kernel against the 64-row split tiles: QKV 6.5 /
+// 15, WO 5.6 / 18, W13 9.1 / 15, W2 10 / 35. The waves of a workgroup share no
+// operand reads, so larger grids keep split_kernel.
+template <int EPI, int IB, int JB, int WK, int D>
+__global__ __launch_bounds__(64 * WK) void split_small_kernel(GemmArgs a, const uint16_t *__restrict__ ap,
+                                                             const uint16_t *__restrict__ bp,
+                                                             const int *__restrict__ aexp, const int *__restrict__ bexp,
+                                                             size_t a_plane, size_t b_plane, int kp, int row_tiles,
+                                                             int col_tiles) {
+  constexpr int BM = 32 * IB, BN = 32 * JB;
+  constexpr int OUT = 16 * IB * JB / WK;  // outputs per thread
+  static_assert(16 * IB * JB % WK == 0 && BM + BN <= 64 * WK, "one exponent and OUT outputs per thread");
+  __shared__ float sums[WK][16 * IB * JB][64];
+  __shared__ int tile_exp[BM + BN];
+  __shared__ bool tile_bad[BM + BN];
+  __shared__ int tile_any;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = lane >> 5, l32 = lane & 31;
+  int rt, ct;
+  xcd_tile(blockIdx.x, row_tiles, col_tiles, rt, ct);
+  const int m0 = rt * BM, n0 = ct * BN;
+  if (tid == 0) tile_any = 0;
+  const int stages = kp / kSplitBK;
+  // Stage-major planes: stage s of a plane starts rows_pad * 32 bytes after s - 1.
+  const size_t a_step = a_plane / stages, b_step = b_plane / stages;
+  const uint16_t *asrc = ap + static_cast<size_t>(m0 + l32) * kSplitBK + 8 * h;
+  const uint16_t *bsrc = bp + static_cast<size_t>(n0 + l32) * kSplitBK + 8 * h;
+  struct Frags {
+    PairFrag a[IB][2], b[JB][2];
+  };
+  auto load = [&](Frags &f, int stage) __attribute__((always_inline)) {
+    const int s = stage < stages ? stage : stages - 1;
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+#pragma unroll
+      for (int i = 0; i < IB; i++)
+        f.a[i][p].u = *reinterpret_cast<const uint4 *>(asrc + p * a_plane + s * a_step + 32 * i * kSplitBK);
+#pragma unroll
+      for (int j = 0; j < JB; j++)
+        f.b[j][p].u = *reinterpret_cast<const uint4 *>(bsrc + p * b_plane + s * b_step + 32 * j * kSplitBK);
+    }
+  };
+  v16f acc[IB][JB];
+#pragma unroll
+  for (int i = 0; i < IB; i++)
+#pragma unroll
+    for (int j = 0; j < JB; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+  Frags f[D];
+#pragma unroll
+  for (int d = 0; d < D; d++) load(f[d], wave + WK * d);
+  for (int st = wave; st < stages; st += WK * D) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      if (st + WK * d < stages) {
+        constexpr int pa[3] = {1, 0, 0}, pb[3] = {0, 1, 0};  // smallest first, as split_kernel
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+          for (int i = 0; i < IB; i++)
+#pragma unroll
+            for (int j = 0; j < JB; j++)
+              acc[i][j] =
+                  __builtin_amdgcn_mfma_f32_32x32x16_f16(f[d].a[i][pa[q]].v, f[d].b[j][pb[q]].v, acc[i][j], 0, 0, 0);
+        load(f[d], st + WK * (d + D));
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < IB; i++)
+#pragma unroll
+    for (int j = 0; j < JB; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) sums[wave][(i * JB + j) * 16 + r][lane] = acc[i][j][r];
+  __syncthreads();
+  if (tid < BM + BN) {
+    const int e = tid < BM ? aexp[m0 + tid] : bexp[n0 + tid - BM];
+    const bool bad = e >= kPairNonfinite / 2;
+    tile_exp[tid] = bad ? e - kPairNonfinite : e;
+    tile_bad[tid] = bad;
+    if (bad) tile_any = 1;
+  }
+  __syncthreads();
+  const bool any = tile_any != 0;
+#pragma unroll
+  for (int o = 0; o < OUT; o++) {
+    const int q = wave * OUT + o, i = q / (16 * JB), j = q / 16 % JB, r = q % 16;
+    float v = sums[0][q][lane];
+#pragma unroll
+    for (int w = 1; w < WK; w++) v += sums[w][q][lane];
+    // D layout of 32x32: column = lane % 32, row = 8 (r / 4) + 4 (lane / 32) + r % 4.
+    const int lr = 32 * i + 8 * (r / 4) + 4 * h + (r % 4), lc = 32 * j + l32;
+    v = __builtin_ldexpf(v, tile_exp[lr] + tile_exp[BM + lc] - 30);
+    const int row = m0 + lr, col = n0 + lc;
+    if (any && row < a.m && col < a.n &&
+        (tile_bad[lr] || tile_bad[BM + lc] || (EPI == FOCR_EPI_GLU && tile_bad[BM + (lc ^ 1)])))
+      v = chain_output(a, row, col);
+    const float partner = EPI == FOCR_EPI_GLU ? __shfl_xor(v, 1) : 0.0f;
+    emit<EPI>(a, row, col, v, partner);
+  }
+}
+
 // The row exponents and FP16-pair planes of src [r][c] (rows padded to
 // r_pad, a multiple of 128; columns to kp).
 void pair_operand(hipStream_t stream, const float *src, size_t r, size_t c, const float *rs, int *exps, uint16_t *dst,
@@ -1275,6 +1386,41 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
                            bexp, a_plane, b_plane, k32, rtiles, ctiles);
     }
   };
+  // By 32 x 32 blocks of output (us, this form and its neighbours): 120 (WO,
+  // m = 144) 32 x 32 5.7, 32 x 64 7.0; 288 (W13, 48) 32 x 64 6.5, 32 x 32 8.0;
+  // 312 (W2, 400) 32 x 64 13.9, 32 x 32 16.4, 64 x 64 18.3; 528 (W2, 700) 64 x 64
+  // 18.8, 32 x 64 22+; 1,872 (W13, 400) 64 x 64 17.2, split_kernel 17.7; 3,000
+  // (WO, 4,000) 29.1 and 30.3; 3,008 (QKV, 1,501) 24.2 and 24.0; 3,168 (W13, 700)
+  // 29.4 and 24.2.
+  auto launch_small = [&](auto ib, auto jb, auto wk, auto depth) {
+    constexpr int IB = decltype(ib)::value, JB = decltype(jb)::value, WK = decltype(wk)::value, D = decltype(depth)::value;
+    const int rt = static_cast<int>((rows + 32 * IB - 1) / (32 * IB)), ct = static_cast<int>(n_pad / (32 * JB));
+    const dim3 grid(static_cast<unsigned>(rt * ct));
+    if (epilogue == FOCR_EPI_GLU)
+      hipLaunchKernelGGL((split_small_kernel<FOCR_EPI_GLU, IB, JB, WK, D>), grid, dim3(64 * WK), 0, ctx->stream, a, ap, bp,
+                         aexp, bexp, a_plane, b_plane, k32, rt, ct);
+    else if (epilogue == FOCR_EPI_ADD)
+      hipLaunchKernelGGL((split_small_kernel<FOCR_EPI_ADD, IB, JB, WK, D>), grid, dim3(64 * WK), 0, ctx->stream, a, ap, bp,
+                         aexp, bexp, a_plane, b_plane, k32, rt, ct);
+    else
+      hipLaunchKernelGGL((split_small_kernel<FOCR_EPI_STORE, IB, JB, WK, D>), grid, dim3(64 * WK), 0, ctx->stream, a, ap,
+                         bp, aexp, bexp, a_plane, b_plane, k32, rt, ct);
+  };
+  using std::integral_constant;
+  const size_t blocks = ((rows + 31) / 32) * ((lin->n + 31) / 32);
+  if (blocks <= 3000) {
+    if (blocks <= 160)
+      launch_small(integral_constant<int, 1>(), integral_constant<int, 1>(), integral_constant<int, 8>(),
+                   integral_constant<int, 4>());
+    else if (blocks <= 420)
+      launch_small(integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 8>(),
+                   integral_constant<int, 3>());
+    else
+      launch_small(integral_constant<int, 2>(), integral_constant<int, 2>(), integral_constant<int, 4>(),
+                   integral_constant<int, 3>());
+    FOCR_HIP_CHECK(hipGetLastError());
+    return FOCR_OK;
+  }
   // 128-row tiles fill 512 workgroup slots (two per compute unit, by VGPRs).
   // Fewer tiles than that run as 64-row tiles (twice as many, half the
   // work each); when the 128-row tiles' last round would be at most half

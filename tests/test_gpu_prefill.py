@@ -189,6 +189,13 @@ def test_f32_split_within_fp32_tolerance(fh, m, k, n):
     assert_bitwise(add, (base + got).astype(np.float32), "add of store")
 
 
+# The small-grid forms (32 x 32, 32 x 64 and 64 x 64 outputs by the number of
+# 32 x 32 blocks): fewer k stages than a workgroup has waves, ragged edges.
+@pytest.mark.parametrize("m,k,n", [(33, 40, 50), (161, 2304, 1000), (700, 300, 700), (1000, 96, 2046)])
+def test_f32_split_small_grids(fh, m, k, n):
+    test_f32_split_within_fp32_tolerance(fh, m, k, n)
+
+
 def test_f32_split_error_is_fp32_level(fh):
     # Against the exact (f64) product: the split kernel's error is of the
     # FP32 matrix-core kernel's order (each pair holds its value to 2^-22, the
@@ -213,7 +220,7 @@ def test_f32_split_tile_heights(fh, m):
     # Launch shapes of the FP16-pair kernel: 2,048 rows x 4,096 outputs fill
     # one whole round of 128-row tiles; 2,176 rows leave a last round at most
     # half full, which runs as 64-row tiles after the whole rounds (the small
-    # shapes above run as 64-row tiles only). Every output within the FP32
+    # shapes above take the small-grid forms). Every output within the FP32
     # bound, Store and Add.
     k, n = 256, 4096
     oracle.set_threads(oracle_threads())
