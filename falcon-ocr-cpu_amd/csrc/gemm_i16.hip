@@ -29,6 +29,8 @@
 // epilogue it runs about 25 % faster, without the products about 15 %; the
 // operand copies (L2 -> LDS, about 1 GB per 6544 x 1024 x 4096 call) and the
 // per-group barrier take the rest.
+#include <type_traits>
+
 #include "focr_internal.hpp"
 
 namespace focr {
@@ -193,6 +195,28 @@ __device__ __forceinline__ void tile_of(int b, int row_tiles, int col_tiles, int
   rt = panel * kPanel + rem % rows;
 }
 
+// One output: its exception FMAs (ascending columns), then the epilogue.
+// Whole waves call it (Glu exchanges neighbouring columns between lanes).
+template <int EPI>
+__device__ __forceinline__ void emit(float v, int row, int col, int m, int n, const float *__restrict__ exc_inputs,
+                                     const float *__restrict__ exc_vals, int n_exc, float *__restrict__ out) {
+  const bool live = row < m && col < n;
+  if (n_exc && live)
+    for (int e = 0; e < n_exc; e++)
+      v = fmaf_(exc_inputs[static_cast<size_t>(row) * n_exc + e], exc_vals[static_cast<size_t>(col) * n_exc + e], v);
+  if constexpr (EPI == FOCR_EPI_GLU) {
+    const float up = __shfl_xor(v, 1);
+    if (live && (col & 1) == 0) out[static_cast<size_t>(row) * (n / 2) + col / 2] = squared_relu_glu(v, up);
+  } else if constexpr (EPI == FOCR_EPI_ADD) {
+    if (live) {
+      float *dst = out + static_cast<size_t>(row) * n + col;
+      *dst = *dst + v;
+    }
+  } else {
+    if (live) out[static_cast<size_t>(row) * n + col] = v;
+  }
+}
+
 // 64 x BN outputs per workgroup of BN / 16 waves; wave (wm, wn) holds 32
 // rows x 32 columns, 2 row blocks x 2 column blocks of 16 x 16. A wider tile
 // moves fewer operand bytes per output (the activation planes are copied once
@@ -341,36 +365,103 @@ void gemm_kernel(const int8_t *__restrict__ a_tiles, const float *__restrict__ s
   // The repeated copies must land before the workgroup's LDS is released.
   __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
 
-  // Exception FMAs (ascending columns), then the epilogue.
 #pragma unroll
-  for (int i = 0; i < RW; i++) {
-    const int row_base = (mb0 + wm * RW + i) * 16 + 4 * quad;
+  for (int i = 0; i < RW; i++)
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const int col = (nb0 + wn * 2 + j) * 16 + col_in;
-      const bool col_ok = col < n;
+    for (int j = 0; j < 2; j++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int row = row_base + r;
-        float v = acc[i][j][r];
-        if (n_exc && col_ok && row < m)
-          for (int e = 0; e < n_exc; e++)
-            v = fmaf_(exc_inputs[static_cast<size_t>(row) * n_exc + e], exc_vals[static_cast<size_t>(col) * n_exc + e], v);
-        if constexpr (EPI == FOCR_EPI_GLU) {
-          const float up = __shfl_xor(v, 1);
-          if (col_ok && row < m && (col & 1) == 0)
-            out[static_cast<size_t>(row) * (n / 2) + col / 2] = squared_relu_glu(v, up);
-        } else if constexpr (EPI == FOCR_EPI_ADD) {
-          if (col_ok && row < m) {
-            float *dst = out + static_cast<size_t>(row) * n + col;
-            *dst = *dst + v;
+      for (int r = 0; r < 4; r++)
+        emit<EPI>(acc[i][j][r], (mb0 + wm * RW + i) * 16 + 4 * quad + r, (nb0 + wn * 2 + j) * 16 + col_in, m, n,
+                  exc_inputs, exc_vals, n_exc, out);
+}
+
+// Small grids: RB x CB blocks of 16 x 16 outputs per wave, WAVES such waves
+// side by side in a workgroup (columns), every operand loaded straight into
+// registers D groups ahead (a block of a group is one contiguous 1 KB run in
+// operand order), no LDS and no barrier. Per output the same integers and the
+// same chain over ascending groups as gemm_kernel.
+// Bound: latency. With few tiles gemm_kernel's workgroups wait for each
+// group's copies behind one barrier per group (0.5 us a group); here a group
+// costs a wave its two dependent products and the FP32 step.
+template <int EPI, int RB, int CB, int WAVES, int D>
+__global__ __launch_bounds__(64 * WAVES) void gemm_small_kernel(
+    const int8_t *__restrict__ a_tiles, const float *__restrict__ steps, const float *__restrict__ exc_inputs,
+    const int8_t *__restrict__ b_tiles, const int32_t *__restrict__ wsum, const float *__restrict__ sw,
+    const float *__restrict__ exc_vals, int n_exc, int m, int n, int groups, int row_blocks, int m_pad, int row_tiles,
+    int col_tiles, float *__restrict__ out) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int quad = lane >> 4, col_in = lane & 15;
+  int rt, ct;
+  tile_of(blockIdx.x, row_tiles, col_tiles, rt, ct);
+  const int mb0 = rt * RB, nb0 = (ct * WAVES + wave) * CB, col_blocks = n / 16;
+  if (nb0 >= col_blocks) return;
+  struct Group {
+    v4i hi[RB], lo[RB], b[CB];
+    float4 sa[RB];
+    int32_t ws[CB];
+    float sw[CB];
+  };
+  auto load = [&](Group &f, int group) __attribute__((always_inline)) {
+    const size_t g = group < groups ? group : groups - 1;
+#pragma unroll
+    for (int i = 0; i < RB; i++) {
+      const int mb = mb0 + i < row_blocks ? mb0 + i : row_blocks - 1;
+      const v4i *src = reinterpret_cast<const v4i *>(a_tiles + (g * row_blocks + mb) * 2048);
+      f.hi[i] = src[lane];
+      f.lo[i] = src[64 + lane];
+      f.sa[i] = *reinterpret_cast<const float4 *>(steps + g * m_pad + mb * 16 + 4 * quad);
+    }
+#pragma unroll
+    for (int j = 0; j < CB; j++) {
+      const int nb = nb0 + j < col_blocks ? nb0 + j : col_blocks - 1;
+      f.b[j] = reinterpret_cast<const v4i *>(b_tiles + (g * col_blocks + nb) * 1024)[lane];
+      f.ws[j] = wsum[g * n + nb * 16 + col_in];
+      f.sw[j] = sw[g * n + nb * 16 + col_in];
+    }
+  };
+  float acc[RB][CB][4];
+#pragma unroll
+  for (int i = 0; i < RB; i++)
+#pragma unroll
+    for (int j = 0; j < CB; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[i][j][r] = 0.0f;
+  Group f[D];
+#pragma unroll
+  for (int d = 0; d < D; d++) load(f[d], d);
+  for (int g = 0; g < groups; g += D) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      if (g + d < groups) {
+#pragma unroll
+        for (int i = 0; i < RB; i++)
+#pragma unroll
+          for (int j = 0; j < CB; j++) {
+            const v4i zero = {0, 0, 0, 0};
+            const v4i hsum = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[d].hi[i], f[d].b[j], zero, 0, 0, 0);
+            v4i c;
+#pragma unroll
+            for (int r = 0; r < 4; r++) c[r] = (hsum[r] << 8) + f[d].ws[j];
+            const v4i sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[d].lo[i], f[d].b[j], c, 0, 0, 0);
+            const float sa[4] = {f[d].sa[i].x, f[d].sa[i].y, f[d].sa[i].z, f[d].sa[i].w};
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const float scale = f[d].sw[j] * sa[r];
+              acc[i][j][r] = fmaf_(static_cast<float>(sum[r]), scale, acc[i][j][r]);
+            }
           }
-        } else {
-          if (col_ok && row < m) out[static_cast<size_t>(row) * n + col] = v;
-        }
+        load(f[d], g + d + D);
       }
     }
   }
+#pragma unroll
+  for (int i = 0; i < RB; i++)
+#pragma unroll
+    for (int j = 0; j < CB; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        emit<EPI>(acc[i][j][r], (mb0 + i) * 16 + 4 * quad + r, (nb0 + j) * 16 + col_in, m, n, exc_inputs, exc_vals, n_exc,
+                  out);
 }
 
 }  // namespace
@@ -396,6 +487,46 @@ int launch_prefill_i16(Ctx *ctx, const Linear *lin, const float *x, size_t rows,
                      row_scale, lin->exc_index, static_cast<int>(lin->n_exc), a_tiles, steps, exc_inputs,
                      static_cast<int>(m_pad));
   FOCR_HIP_CHECK(hipGetLastError());
+  // By 16 x 16 blocks of output, against the chip's 1,024 SIMDs (us, this form
+  // and its neighbours, quantizer not counted): 432 (WO, m = 144) 16 x 16 per wave
+  // 4.5, 16 x 32 5.8, gemm_kernel 10; 864 (W13, 48) 4.4, 5.0; 2,592 (W13, 144)
+  // 16 x 32 7.1, 16 x 16 8.4, 32 x 32 8.4, gemm_kernel 9.7; 3,024 (W2, 1,000) 14.5,
+  // 18.5, 18.2, 20; 4,512 (W2, 1,501) 32 x 32 20.5, 16 x 32 21.0, gemm_kernel 23;
+  // 7,200 (W13, 400) 32 x 32 11.9, gemm_kernel 13.8; 7,536 (W2, 2,500) 24.9 and
+  // 23.4; 8,064 (QKV, 1,000) 12.3 and 11.3: larger grids share operands in LDS.
+  const size_t blocks = (m + 15) / 16 * (n / 16);
+  if (blocks <= 7400) {
+    auto launch = [&](auto epi, auto rb, auto cb, auto wv, auto depth) {
+      constexpr int E = decltype(epi)::value, RB = decltype(rb)::value, CB = decltype(cb)::value;
+      constexpr int WV = decltype(wv)::value, D = decltype(depth)::value;
+      const int rt = static_cast<int>((m + 16 * RB - 1) / (16 * RB));
+      const int ct = static_cast<int>((n / 16 + CB * WV - 1) / (CB * WV));
+      hipLaunchKernelGGL((gemm_small_kernel<E, RB, CB, WV, D>), dim3(static_cast<unsigned>(rt * ct)), dim3(64 * WV), 0,
+                         ctx->stream, a_tiles, steps, exc_inputs, lin->i16_b, lin->i16_wsum, lin->i16_sw, lin->exc_vals,
+                         static_cast<int>(lin->n_exc), static_cast<int>(m), static_cast<int>(n),
+                         static_cast<int>(groups), static_cast<int>(row_blocks), static_cast<int>(m_pad), rt, ct, out);
+    };
+    using std::integral_constant;
+    auto pick = [&](auto epi) {
+      if (blocks <= 1000)
+        launch(epi, integral_constant<int, 1>(), integral_constant<int, 1>(), integral_constant<int, 1>(),
+               integral_constant<int, 4>());
+      else if (blocks <= 4000)
+        launch(epi, integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 2>(),
+               integral_constant<int, 3>());
+      else
+        launch(epi, integral_constant<int, 2>(), integral_constant<int, 2>(), integral_constant<int, 2>(),
+               integral_constant<int, 3>());
+    };
+    if (epilogue == FOCR_EPI_GLU)
+      pick(integral_constant<int, FOCR_EPI_GLU>());
+    else if (epilogue == FOCR_EPI_ADD)
+      pick(integral_constant<int, FOCR_EPI_ADD>());
+    else
+      pick(integral_constant<int, FOCR_EPI_STORE>());
+    FOCR_HIP_CHECK(hipGetLastError());
+    return FOCR_OK;
+  }
   // 128-column tiles where n gives at least 16 of them (fewer operand bytes
   // per output: +5 % on 1024 -> 4096), 64-column ones for narrow outputs
   // (n = 768: the wider tiles leave too few workgroups).

@@ -43,6 +43,15 @@ def test_i16_panels_bitwise_every_epilogue(fh, m, k, n):
                    oracle.i16_gemm(a, m, k, codes, scales, n, row_scale=rs, epilogue=oracle.ADD, out=base), "add")
 
 
+# The small-grid forms (16 x 16, 16 x 32 and 32 x 32 outputs per wave by the
+# number of 16 x 16 blocks) and the LDS tiles above them, 64 and 128 columns
+# wide, with ragged rows and odd column-block counts.
+@pytest.mark.parametrize("m,k,n", [(9, 64, 32), (33, 320, 1056), (130, 192, 2208), (301, 256, 4128), (2500, 128, 800),
+                                   (1010, 192, 2080)])
+def test_i16_tile_forms_are_bitwise_the_panels(fh, m, k, n):
+    test_i16_panels_bitwise_every_epilogue(fh, m, k, n)
+
+
 @pytest.mark.parametrize("m,k,n", [(13, 768, 64), (50, 2304, 64), (97, 1024, 32)])
 def test_i16_exception_columns(fh, m, k, n):
     # panel_i16/tests.rs:156-227: two pairs share a group; huge inputs there.
