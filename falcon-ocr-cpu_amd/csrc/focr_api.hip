@@ -164,11 +164,14 @@ int focr_ctx_create(int device, focr_ctx **out) {
     return set_error(FOCR_E_HIP, std::string("hipEventCreate: ") + hipGetErrorString(err));
   }
   err = hipMalloc(&ctx->rms_dev, 8 * sizeof(float));
+  if (err == hipSuccess)
+    err = hipHostMalloc(reinterpret_cast<void **>(&ctx->flags), 16 * sizeof(uint32_t), hipHostMallocDefault);
   if (err != hipSuccess) {
+    if (ctx->rms_dev) (void)hipFree(ctx->rms_dev);
     (void)hipEventDestroy(ctx->order);
     (void)hipStreamDestroy(ctx->own);
     delete ctx;
-    return set_error(FOCR_E_HIP, std::string("hipMalloc: ") + hipGetErrorString(err));
+    return set_error(FOCR_E_HIP, std::string("context buffers: ") + hipGetErrorString(err));
   }
   *out = reinterpret_cast<focr_ctx *>(ctx);
   return FOCR_OK;
@@ -182,6 +185,7 @@ int focr_ctx_destroy(focr_ctx *handle) {
   if (ctx->scratch) FOCR_HIP_CHECK(hipFree(ctx->scratch));
   if (ctx->argmax_dev) FOCR_HIP_CHECK(hipFree(ctx->argmax_dev));
   if (ctx->rms_dev) FOCR_HIP_CHECK(hipFree(ctx->rms_dev));
+  if (ctx->flags) FOCR_HIP_CHECK(hipHostFree(ctx->flags));
   FOCR_HIP_CHECK(hipEventDestroy(ctx->order));
   FOCR_HIP_CHECK(hipStreamDestroy(ctx->own));
   delete ctx;

@@ -42,6 +42,7 @@ struct Ctx {
   uint32_t *argmax_dev = nullptr;  // [2 * rows] result words for focr_argmax
   size_t argmax_rows = 0;
   float *rms_dev = nullptr;  // [8] row scales of a decode GEMV whose width has no in-kernel rms_norm
+  uint32_t *flags = nullptr;  // [16] words of pinned host memory that kernels write and a synchronous call reads
   hipEvent_t order = nullptr;  // orders a new stream after the old one (focr_ctx_set_stream)
 };
 

@@ -35,7 +35,9 @@
 // there. Roofline: HBM; bytes per call = the visible
 // records (Q8: 176 bytes per group and prefix position, 8 groups = 1,408
 // bytes per position against 6,144 for the FP32 compact cache).
+#include <atomic>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "decode_common.hpp"
@@ -81,6 +83,8 @@ float *noalloc_scratch(int device) {
 }
 }  // namespace
 
+inline const hipStream_t kNoStream = reinterpret_cast<hipStream_t>(~uintptr_t(0));
+
 struct KvSplit {
   int bits = 8;
   int n_heads = 0, n_kv = 0;
@@ -88,8 +92,15 @@ struct KvSplit {
   size_t record_bytes = 0, tail_bytes = 0;
   unsigned char *records = nullptr;  // [n_kv][prefix_len][record_bytes]
   unsigned char *tail = nullptr;     // [n_kv][capacity - prefix_len][tail_bytes]
-  uint32_t *error = nullptr;         // seal's refusal flags
+  size_t records_alloc = 0, tail_alloc = 0;  // bytes allocated, at least what the current sizes need
   size_t device_bytes = 0;
+  // The first stream that used this cache since it was sealed (kNoStream:
+  // none), and whether there is work on it that this stream does not order
+  // (another stream's, or a capture's, which may be replayed anywhere): what
+  // focr_kv_reseal has to wait for. Atomic: contexts may read one cache from
+  // several threads.
+  std::atomic<hipStream_t> stream{kNoStream};
+  std::atomic<bool> spread{false};
   bool fast_exp = false;  // SplitPrefix::fast_exp (kv.rs:168-170)
 };
 
@@ -161,7 +172,7 @@ enum : uint32_t { kErrPair = 1, kErrNonFinite = 2, kErrOverflow = 4 };
 struct SealArgs {
   const float *k, *v;
   unsigned char *records;
-  uint32_t *error;
+  uint32_t *error;  // [3], pinned host memory: one word per refusal, set to 1
   int prefix_len, n_heads, n_kv, record_bytes;
 };
 
@@ -208,7 +219,9 @@ __global__ __launch_bounds__(256) void seal_kernel(SealArgs a, long pass) {
       if (!__builtin_isfinite(static_cast<float>(code) * bf16_widen(stored))) err |= kErrOverflow;
     }
   }
-  if (err) atomicOr(a.error, err);
+  if (err & kErrPair) a.error[0] = 1;
+  if (err & kErrNonFinite) a.error[1] = 1;
+  if (err & kErrOverflow) a.error[2] = 1;
 }
 
 struct AppendArgs {
@@ -1023,6 +1036,69 @@ SplitDecArgs split_args(const KvSplit *s, const float *q) {
   return a;
 }
 
+// Notes the stream of a call on the cache.
+void touch(const KvSplit *cs, const Ctx *ctx) {
+  KvSplit *s = const_cast<KvSplit *>(cs);
+  if (s->spread.load(std::memory_order_relaxed)) return;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) (void)hipGetLastError();
+  hipStream_t first = kNoStream;
+  const bool same = s->stream.compare_exchange_strong(first, ctx->stream) || first == ctx->stream;
+  if (!same || capture != hipStreamCaptureStatusNone) s->spread.store(true);
+}
+
+// Seals the prefix into the handle's buffers, which grow when they are too
+// small. A page's layers reseal the same handle, so a prefill allocates and
+// frees nothing: the three allocations, their frees (each waits for the
+// device), a clear and a pageable copy of the error word had cost about 60 us
+// a layer. The kernel reports refusals in the context's pinned words.
+int seal_into(Ctx *ctx, KvSplit *s, const float *prefix_k, const float *v, size_t prefix_len, size_t capacity) {
+  s->prefix_len = prefix_len;
+  s->capacity = capacity;
+  s->tail_len = 0;
+  s->fast_exp = false;
+  const size_t cb = s->bits / 8;
+  s->record_bytes = (kRecord * cb + 10 + 15) / 16 * 16;
+  s->tail_bytes = (kTail * cb + 8 + 15) / 16 * 16;
+  const size_t rec_total = s->n_kv * prefix_len * s->record_bytes;
+  const size_t tail_total = s->n_kv * (capacity - prefix_len) * s->tail_bytes;
+  auto grow = [](unsigned char **buffer, size_t *have, size_t need) {
+    if (need <= *have) return hipSuccess;
+    if (*buffer) (void)hipFree(*buffer);
+    *buffer = nullptr;
+    *have = 0;
+    const hipError_t e = hipMalloc(reinterpret_cast<void **>(buffer), need);
+    if (e == hipSuccess) *have = need;
+    return e;
+  };
+  hipError_t e = grow(&s->records, &s->records_alloc, rec_total);
+  if (e == hipSuccess) e = grow(&s->tail, &s->tail_alloc, tail_total);
+  if (e != hipSuccess) return set_error(FOCR_E_HIP, std::string("focr_kv_seal: ") + hipGetErrorString(e));
+  s->device_bytes = rec_total + tail_total;
+  volatile uint32_t *flags = ctx->flags;
+  flags[0] = flags[1] = flags[2] = 0;
+  SealArgs a{prefix_k, v, s->records, ctx->flags, static_cast<int>(prefix_len), s->n_heads, s->n_kv,
+             static_cast<int>(s->record_bytes)};
+  const long nrec = static_cast<long>(s->n_kv) * prefix_len;
+  const long pass = (nrec + kSealPer - 1) / kSealPer;
+  const dim3 grid(static_cast<unsigned>((pass * kRecord + 255) / 256));
+  static_assert(kRecord % 32 == 0 && kTail % 64 == 0, "blocks are whole half-waves");
+  if (s->bits == 8)
+    hipLaunchKernelGGL(seal_kernel<int8_t>, grid, dim3(256), 0, ctx->stream, a, pass);
+  else
+    hipLaunchKernelGGL(seal_kernel<int16_t>, grid, dim3(256), 0, ctx->stream, a, pass);
+  e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  if (e != hipSuccess) return set_error(FOCR_E_HIP, std::string("focr_kv_seal: ") + hipGetErrorString(e));
+  if (flags[0])
+    return set_error(FOCR_E_VALUE, "temporal keys differ inside GQA pair; refusing illegal sharing");
+  if (flags[1]) return set_error(FOCR_E_VALUE, "nonfinite or incomplete KV group");
+  if (flags[2])
+    return set_error(FOCR_E_VALUE, s->bits == 8 ? "Q8 KV conversion overflow" : "Q16 KV conversion overflow");
+  touch(s, ctx);
+  return FOCR_OK;
+}
+
 }  // namespace
 }  // namespace focr
 
@@ -1043,52 +1119,38 @@ int focr_kv_seal(focr_ctx *handle, int bits, const float *prefix_k, const float 
   FOCR_REQUIRE(prefix_len * n_kv_heads * kRecord / 256 < (size_t(1) << 31), FOCR_E_SHAPE,
                "split prefix too long for one seal launch");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  KvSplit *s = new KvSplit();
+  KvSplit *s = new (std::nothrow) KvSplit();
+  FOCR_REQUIRE(s, FOCR_E_ARG, "focr_kv_seal: out of host memory");
   s->bits = bits;
   s->n_heads = static_cast<int>(n_heads);
   s->n_kv = static_cast<int>(n_kv_heads);
-  s->prefix_len = prefix_len;
-  s->capacity = capacity;
-  const size_t cb = bits / 8;
-  s->record_bytes = (kRecord * cb + 10 + 15) / 16 * 16;
-  s->tail_bytes = (kTail * cb + 8 + 15) / 16 * 16;
-  const size_t rec_total = n_kv_heads * prefix_len * s->record_bytes;
-  const size_t tail_total = n_kv_heads * (capacity - prefix_len) * s->tail_bytes;
-  hipError_t e = hipMalloc(reinterpret_cast<void **>(&s->records), rec_total);
-  if (e == hipSuccess && tail_total) e = hipMalloc(reinterpret_cast<void **>(&s->tail), tail_total);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&s->error), sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMemsetAsync(s->error, 0, sizeof(uint32_t), ctx->stream);
-  if (e != hipSuccess) {
+  const int rc = seal_into(ctx, s, prefix_k, v, prefix_len, capacity);
+  if (rc != FOCR_OK) {
     focr_kv_free(reinterpret_cast<focr_kv_split *>(s));
-    return set_error(FOCR_E_HIP, std::string("focr_kv_seal: ") + hipGetErrorString(e));
-  }
-  s->device_bytes = rec_total + tail_total;
-  SealArgs a{prefix_k, v, s->records, s->error, static_cast<int>(prefix_len), s->n_heads, s->n_kv,
-             static_cast<int>(s->record_bytes)};
-  const long nrec = static_cast<long>(n_kv_heads) * prefix_len;
-  const long pass = (nrec + kSealPer - 1) / kSealPer;
-  const dim3 grid(static_cast<unsigned>((pass * kRecord + 255) / 256));
-  static_assert(kRecord % 32 == 0 && kTail % 64 == 0, "blocks are whole half-waves");
-  if (bits == 8)
-    hipLaunchKernelGGL(seal_kernel<int8_t>, grid, dim3(256), 0, ctx->stream, a, pass);
-  else
-    hipLaunchKernelGGL(seal_kernel<int16_t>, grid, dim3(256), 0, ctx->stream, a, pass);
-  uint32_t err = 0;
-  e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(&err, s->error, sizeof(err), hipMemcpyDeviceToHost, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  if (e != hipSuccess) {
-    focr_kv_free(reinterpret_cast<focr_kv_split *>(s));
-    return set_error(FOCR_E_HIP, std::string("focr_kv_seal: ") + hipGetErrorString(e));
-  }
-  if (err) {
-    focr_kv_free(reinterpret_cast<focr_kv_split *>(s));
-    if (err & kErrPair) return set_error(FOCR_E_VALUE, "temporal keys differ inside GQA pair; refusing illegal sharing");
-    if (err & kErrNonFinite) return set_error(FOCR_E_VALUE, "nonfinite or incomplete KV group");
-    return set_error(FOCR_E_VALUE, bits == 8 ? "Q8 KV conversion overflow" : "Q16 KV conversion overflow");
+    return rc;
   }
   *out = reinterpret_cast<focr_kv_split *>(s);
   return FOCR_OK;
+}
+
+int focr_kv_reseal(focr_ctx *handle, focr_kv_split *kv, const float *prefix_k, const float *v, size_t prefix_len,
+                   size_t capacity) {
+  Ctx *ctx = reinterpret_cast<Ctx *>(handle);
+  KvSplit *s = reinterpret_cast<KvSplit *>(kv);
+  FOCR_REQUIRE(ctx && s && prefix_k && v, FOCR_E_ARG, "focr_kv_reseal: null argument");
+  FOCR_REQUIRE(prefix_len > 0 && capacity >= prefix_len && capacity < (size_t(1) << 30), FOCR_E_SHAPE,
+               "invalid split-prefix capacity");
+  FOCR_REQUIRE(prefix_len * s->n_kv * kRecord / 256 < (size_t(1) << 31), FOCR_E_SHAPE,
+               "split prefix too long for one seal launch");
+  FOCR_HIP_CHECK(hipSetDevice(ctx->device));
+  // Work on the old records that this stream does not order before the seal.
+  const hipStream_t used = s->stream.load();
+  if (s->spread.load() || (used != kNoStream && used != ctx->stream)) FOCR_HIP_CHECK(hipDeviceSynchronize());
+  s->stream.store(kNoStream);
+  s->spread.store(false);
+  const int rc = seal_into(ctx, s, prefix_k, v, prefix_len, capacity);
+  if (rc != FOCR_OK) s->prefix_len = s->capacity = s->tail_len = 0;  // nothing to attend over or append to
+  return rc;
 }
 
 int focr_kv_append(focr_ctx *handle, focr_kv_split *kv, const float *k, const float *v, size_t rows) {
@@ -1098,6 +1160,7 @@ int focr_kv_append(focr_ctx *handle, focr_kv_split *kv, const float *k, const fl
   if (rows == 0) return FOCR_OK;
   FOCR_REQUIRE(s->prefix_len + s->tail_len + rows <= s->capacity, FOCR_E_SHAPE, "split tail capacity");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
+  touch(s, ctx);
   AppendArgs a{k, v, s->tail, s->n_kv, static_cast<int>(s->capacity - s->prefix_len), static_cast<int>(s->tail_len),
                static_cast<int>(rows), static_cast<int>(s->tail_bytes)};
   const int threads = static_cast<int>(rows) * s->n_kv * kTail;
@@ -1119,6 +1182,7 @@ int focr_kv_qkv_rows(focr_ctx *handle, focr_kv_split *kv, const float *qkv, size
   FOCR_REQUIRE(rows <= 8, FOCR_E_SHAPE, "decode takes 1..=8 rows");
   FOCR_REQUIRE(s->prefix_len + s->tail_len + rows <= s->capacity, FOCR_E_SHAPE, "split tail capacity");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
+  touch(s, ctx);
   RowAppendArgs a{qkv, rope, q, s->tail, s->n_heads, s->n_kv, static_cast<int>(s->capacity - s->prefix_len),
                   static_cast<int>(s->tail_len), static_cast<int>(s->tail_bytes)};
   if (s->bits == 8)
@@ -1140,6 +1204,7 @@ int focr_kv_decode_row(focr_ctx *handle, focr_kv_split *kv, const float *qkv, co
   FOCR_REQUIRE(s->prefix_len + s->tail_len + 1 <= s->capacity, FOCR_E_SHAPE, "split tail capacity");
   FOCR_REQUIRE(s->n_heads == 2 * s->n_kv, FOCR_E_SHAPE, "split decode: two query heads per KV head");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
+  touch(s, ctx);
   SplitDecArgs a = split_args(s, nullptr);
   a.last += 1;  // the new row is position prefix_len + tail_len
   a.qkv = qkv;
@@ -1160,6 +1225,7 @@ int focr_kv_attention_decode(focr_ctx *handle, const focr_kv_split *kv, const fl
   FOCR_REQUIRE(rows >= 1 && rows <= 8 && rows <= (s->tail_len > 0 ? s->tail_len : 1), FOCR_E_SHAPE,
                "split decode: 1 to 8 rows, at most the appended positions");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
+  touch(s, ctx);
   const SplitDecArgs a = split_args(s, q);
   const int r = static_cast<int>(rows);
   return s->bits == 8 ? launch_split_rows<int8_t>(ctx, a, r, s->fast_exp, sinks, out, nullptr, 0)
@@ -1174,6 +1240,7 @@ int focr_kv_attention_decode_noalloc(focr_ctx *handle, const focr_kv_split *kv, 
   FOCR_REQUIRE(rows >= 1 && rows <= 8 && rows <= (s->tail_len > 0 ? s->tail_len : 1), FOCR_E_SHAPE,
                "split decode: 1 to 8 rows, at most the appended positions");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
+  touch(s, ctx);
   float *fixed = noalloc_scratch(ctx->device);
   FOCR_REQUIRE(fixed, FOCR_E_HIP, "the no-alloc scratch of this device was not resolved (focr_ctx_create does it)");
   const SplitDecArgs a = split_args(s, q);
@@ -1188,6 +1255,7 @@ int focr_kv_dequantize(focr_ctx *handle, const focr_kv_split *kv, float *prefix_
   FOCR_REQUIRE(ctx && s && prefix_k && values && (generated_k || s->tail_len == 0), FOCR_E_ARG,
                "focr_kv_dequantize: null argument");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
+  touch(s, ctx);
   DequantArgs a{s->records, s->tail, prefix_k, values, generated_k, static_cast<int>(s->prefix_len),
                 static_cast<int>(s->tail_len), static_cast<int>(s->capacity - s->prefix_len), s->n_heads, s->n_kv,
                 static_cast<int>(s->record_bytes), static_cast<int>(s->tail_bytes)};
@@ -1240,7 +1308,6 @@ int focr_kv_free(focr_kv_split *kv) {
   if (!s) return FOCR_OK;
   if (s->records) (void)hipFree(s->records);
   if (s->tail) (void)hipFree(s->tail);
-  if (s->error) (void)hipFree(s->error);
   delete s;
   return FOCR_OK;
 }

@@ -281,6 +281,14 @@ extern "C" {
         head_dim: usize,
         out: *mut *mut focr_kv_split,
     ) -> c_int;
+    pub fn focr_kv_reseal(
+        ctx: *mut focr_ctx,
+        kv: *mut focr_kv_split,
+        prefix_k_dev: *const f32,
+        v_dev: *const f32,
+        prefix_len: usize,
+        capacity: usize,
+    ) -> c_int;
     pub fn focr_kv_append(
         ctx: *mut focr_ctx,
         kv: *mut focr_kv_split,

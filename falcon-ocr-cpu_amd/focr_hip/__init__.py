@@ -78,6 +78,7 @@ SIGNATURES = {
     "focr_attention_prefill_bf16": (_I, [_P, _P, _P, _P, _Z, _Z, _Z, _Z, _Z, _Z, _P, _I, _I, _P]),
     "focr_argmax": (_I, [_P, _P, _Z, _Z, _P]),
     "focr_kv_seal": (_I, [_P, _I, _P, _P, _Z, _Z, _Z, _Z, _Z, ctypes.POINTER(_P)]),
+    "focr_kv_reseal": (_I, [_P, _P, _P, _P, _Z, _Z]),
     "focr_kv_append": (_I, [_P, _P, _P, _P, _Z]),
     "focr_kv_attention_decode": (_I, [_P, _P, _P, _Z, _P, _P]),
     "focr_kv_attention_decode_noalloc": (_I, [_P, _P, _P, _Z, _P, _P]),
@@ -540,6 +541,15 @@ class KvSplit:
         _check(lib().focr_kv_seal(ctx.handle, bits, _dev(prefix_k), _dev(v), prefix_len, capacity, n_heads,
                                   n_kv_heads, 64, ctypes.byref(handle)))
         return cls(handle, bits, n_heads, n_kv_heads, ctx)
+
+    def reseal(self, prefix_k, v, prefix_len: int, capacity: int) -> "KvSplit":
+        """`seal` of another prefix in this cache's buffers, which stay
+        allocated: returns the new cache; this one is freed by it (as `free`
+        leaves it), also when the seal is refused."""
+        handle, self.handle = self.handle, None
+        new = KvSplit(handle, self.bits, self.n_heads, self.n_kv_heads, self.ctx)
+        _check(lib().focr_kv_reseal(self.ctx.handle, handle, _dev(prefix_k), _dev(v), prefix_len, capacity))
+        return new
 
     def append(self, k, v, rows: int) -> None:
         """`push_unique` of `rows` positions: k, v [rows][n_kv_heads][64]."""

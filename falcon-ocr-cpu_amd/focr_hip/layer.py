@@ -121,9 +121,12 @@ class DecoderLayer:
             raise FocrError(-2, "attention image must be inside the prefix")
         ctx = self.ctx
         mark = clock or (lambda stage: None)
-        if self.split is not None:
-            self.split.free()
-            self.split = None
+        # The last prompt's sealed cache is gone; its buffers serve this one's.
+        old, self.split = self.split, None
+        if old is not None and (not old.handle or old.ctx is not ctx
+                                or (old.bits, old.n_heads, old.n_kv_heads) != (self.kv_bits, self.n_heads, self.n_kv_heads)):
+            old.free()
+            old = None
         # The panel path takes more than 8 rows (`panel = rows > 8 && ...`,
         # model/mod.rs:568); shorter prompts run the decode step's GEMVs.
         panel = rows > 8
@@ -152,8 +155,10 @@ class DecoderLayer:
             attn = attention_with(q, self.kv(rows), rows, geometry, self.sinks, options, output=attn, ctx=ctx)
         mark("attention")
         if self.kv_bits != 32:
-            self.split = KvSplit.seal(self.kv_bits, self.prefix_k[:rows], self.v[:rows], rows, self.capacity,
-                                      self.n_heads, self.n_kv_heads, ctx=ctx).set_fast_exp(self.decode_fast_exp)
+            k, v = self.prefix_k[:rows], self.v[:rows]
+            split = (KvSplit.seal(self.kv_bits, k, v, rows, self.capacity, self.n_heads, self.n_kv_heads, ctx=ctx)
+                     if old is None else old.reseal(k, v, rows, self.capacity))
+            self.split = split.set_fast_exp(self.decode_fast_exp)
             mark("seal")
         if panel:
             self.wo.prefill(attn, rows, epilogue=Epilogue.ADD, out=h, kernel=self.projection)

@@ -319,6 +319,14 @@ int focr_argmax(focr_ctx *ctx, const float *logits_dev, size_t rows, size_t voca
 int focr_kv_seal(focr_ctx *ctx, int bits, const float *prefix_k_dev, const float *v_dev,
                  size_t prefix_len, size_t capacity, size_t n_heads, size_t n_kv_heads,
                  size_t head_dim, focr_kv_split **out);
+/* focr_kv_seal into an existing handle (its bits and heads): its old prefix
+ * and tail are dropped, its buffers are kept where they are large enough, so
+ * a session's next page allocates nothing. Waits for work queued on the old
+ * records from other streams or captured graphs. After an error the handle
+ * holds no prefix and may only be resealed or freed. No reference counterpart
+ * (device state). */
+int focr_kv_reseal(focr_ctx *ctx, focr_kv_split *kv, const float *prefix_k_dev, const float *v_dev,
+                   size_t prefix_len, size_t capacity);
 /* SplitPrefix::append / push_unique (src/quant/kv.rs:430-515): appends rows
  * generated positions, one key and one value per KV group (k_dev, v_dev
  * [rows][n_kv_heads][64]: the pair's identical heads once), coded as the

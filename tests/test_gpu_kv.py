@@ -111,6 +111,41 @@ def test_refusals(fh):
     kv.free()
 
 
+@pytest.mark.parametrize("bits", [8, 16])
+def test_reseal_is_bitwise_a_fresh_seal(fh, bits):
+    # One handle through pages of other lengths (its buffers kept, then grown),
+    # with work of another stream on the old records, and a refused page.
+    import torch
+
+    ctx = fh.default_context()
+    kv = None
+    for i, (P, cap) in enumerate([(300, 309), (37, 46), (1000, 1009), (999, 1009)]):
+        k, v = pair_cache(P, N_KV, 50 + i, 2.0)
+        tk, tv = gen.normal((3, N_KV, 64), 1.0, 60 + i), gen.normal((3, N_KV, 64), 1.0, 70 + i)
+        kd, vd = to_dev(k), to_dev(v)
+        old = kv
+        kv = fh.KvSplit.seal(bits, kd, vd, P, cap, N_HEADS, N_KV) if old is None else old.reseal(kd, vd, P, cap)
+        assert old is None or old.handle is None
+        assert kv.info()[:4] == (bits, P, 0, cap) and kv.fast_exp is False
+        kv.set_fast_exp(True).append(to_dev(tk), to_dev(tv), 3)
+        for got, want in zip(kv.dequantize(), oracle_cache(bits, k, v, P, tk, tv, cap)):
+            assert_bitwise(host(got), want)
+        fresh = fh.KvSplit.seal(bits, kd, vd, P, cap, N_HEADS, N_KV)
+        assert kv.info() == fresh.info()[:2] + (3,) + fresh.info()[3:]
+        fresh.free()
+        side = torch.cuda.Stream()
+        ctx.use_stream(side)
+        q, sinks = to_dev(gen.normal((2, N_HEADS, 64), 1.0, 80)), to_dev(gen.uniform(N_HEADS, -2.0, 2.0, 81))
+        side.wait_stream(torch.cuda.current_stream())
+        kv.attention_decode(q, 2, sinks)
+        ctx.use_stream(torch.cuda.current_stream())
+    nan = v.copy()
+    nan[4, 7, 63] = np.nan
+    with pytest.raises(fh.FocrError, match="nonfinite"):
+        kv.reseal(kd, to_dev(nan), P, cap)
+    assert kv.handle is None
+
+
 @pytest.mark.parametrize("fast", [False, True])
 @pytest.mark.parametrize("bits", [8, 16])
 @pytest.mark.parametrize("prefix_len,tail,rows", [(64, 1, 1), (700, 3, 3), (2000, 8, 8), (129, 5, 2)])
