@@ -183,7 +183,7 @@ int focr_ctx_destroy(focr_ctx *handle) {
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
   FOCR_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   if (ctx->scratch) FOCR_HIP_CHECK(hipFree(ctx->scratch));
-  if (ctx->argmax_dev) FOCR_HIP_CHECK(hipFree(ctx->argmax_dev));
+  if (ctx->argmax) FOCR_HIP_CHECK(hipHostFree(ctx->argmax));
   if (ctx->rms_dev) FOCR_HIP_CHECK(hipFree(ctx->rms_dev));
   if (ctx->flags) FOCR_HIP_CHECK(hipHostFree(ctx->flags));
   FOCR_HIP_CHECK(hipEventDestroy(ctx->order));
@@ -646,23 +646,41 @@ int focr_argmax(focr_ctx *handle, const float *logits, size_t rows, size_t vocab
   if (rows == 0) return FOCR_OK;
   FOCR_REQUIRE(logits && tokens, FOCR_E_ARG, "focr_argmax: null buffer");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  if (ctx->argmax_rows < rows) {
-    if (ctx->argmax_dev) {
+  // Parts of at least 4,096 values (one pass of a workgroup's loads), at most
+  // 64 of them, and fewer when the rows fill the chip by themselves.
+  const size_t spread = std::min<size_t>(64, std::max<size_t>(1, 1024 / rows));
+  const size_t parts = std::min(spread, (vocab + 4095) / 4096);
+  const size_t chunk = ((vocab + parts - 1) / parts + 3) / 4 * 4;
+  if (ctx->argmax_parts < rows * parts) {
+    if (ctx->argmax) {
       FOCR_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-      FOCR_HIP_CHECK(hipFree(ctx->argmax_dev));
-      ctx->argmax_dev = nullptr;
+      FOCR_HIP_CHECK(hipHostFree(ctx->argmax));
+      ctx->argmax = nullptr;
+      ctx->argmax_parts = 0;
     }
-    FOCR_HIP_CHECK(hipMalloc(&ctx->argmax_dev, rows * 2 * sizeof(uint32_t)));
-    ctx->argmax_rows = rows;
+    const size_t count = std::max<size_t>(rows * parts, 256);
+    FOCR_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&ctx->argmax), count * sizeof(ArgmaxPart), hipHostMallocDefault));
+    ctx->argmax_parts = count;
   }
-  int rc = launch_argmax(ctx, logits, rows, vocab, ctx->argmax_dev);
+  int rc = launch_argmax(ctx, logits, rows, vocab, static_cast<int>(parts), static_cast<int>(chunk), ctx->argmax);
   if (rc != FOCR_OK) return rc;
-  std::vector<uint32_t> result(rows * 2);
-  FOCR_HIP_CHECK(hipMemcpyAsync(result.data(), ctx->argmax_dev, rows * 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
   FOCR_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   for (size_t r = 0; r < rows; r++) {
-    FOCR_REQUIRE(result[2 * r + 1] == 0, FOCR_E_NONFINITE, "nonfinite or empty logits");
-    tokens[r] = result[2 * r];
+    const volatile ArgmaxPart *part = ctx->argmax + r * parts;
+    float best = 0.0f;
+    int32_t token = -1;
+    bool bad = false;
+    for (size_t p = 0; p < parts; p++) {  // ascending: the first of equal values stays
+      bad |= part[p].nonfinite != 0;
+      const float value = part[p].value;
+      const int32_t index = part[p].index;
+      if (index >= 0 && (token < 0 || value > best)) {
+        best = value;
+        token = index;
+      }
+    }
+    FOCR_REQUIRE(!bad, FOCR_E_NONFINITE, "nonfinite or empty logits");
+    tokens[r] = static_cast<uint32_t>(token);
   }
   return FOCR_OK;
 }

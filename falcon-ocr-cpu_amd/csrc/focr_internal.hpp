@@ -31,6 +31,13 @@ int set_error(int code, const std::string &message);
     if (!(cond)) return ::focr::set_error((code), (msg));                                 \
   } while (0)
 
+// What one workgroup of focr_argmax found in its part of a row.
+struct alignas(16) ArgmaxPart {
+  float value;
+  int32_t index;  // first index of the value, -1: no values
+  uint32_t nonfinite, pad;
+};
+
 // ---- context ---------------------------------------------------------------
 struct Ctx {
   int device = 0;
@@ -39,8 +46,8 @@ struct Ctx {
   // Scratch owned by the context, grown on demand (INT16 activation codes).
   void *scratch = nullptr;
   size_t scratch_bytes = 0;
-  uint32_t *argmax_dev = nullptr;  // [2 * rows] result words for focr_argmax
-  size_t argmax_rows = 0;
+  ArgmaxPart *argmax = nullptr;  // focr_argmax's results, pinned host memory
+  size_t argmax_parts = 0;
   float *rms_dev = nullptr;  // [8] row scales of a decode GEMV whose width has no in-kernel rms_norm
   uint32_t *flags = nullptr;  // [16] words of pinned host memory that kernels write and a synchronous call reads
   hipEvent_t order = nullptr;  // orders a new stream after the old one (focr_ctx_set_stream)
@@ -113,7 +120,7 @@ int launch_attention_split(Ctx *ctx, const float *q, const float *k, const float
 int launch_attention_bf16(Ctx *ctx, const float *q, const float *k, const float *v, size_t query_len,
                           size_t n_heads, size_t n_kv_heads, size_t image_start, size_t image_end,
                           const float *sinks, int softmax, float *out);
-int launch_argmax(Ctx *ctx, const float *logits, size_t rows, size_t vocab, uint32_t *result_dev);
+int launch_argmax(Ctx *ctx, const float *logits, size_t rows, size_t vocab, int parts, int chunk, ArgmaxPart *result);
 int launch_qkv_rows(Ctx *ctx, const float *qkv, size_t rows, const float *rope, size_t n_heads, size_t n_kv_heads,
                     size_t prefix_rows, float *q, float *prefix_k, float *generated_k, float *v);
 int launch_attention_decode(Ctx *ctx, const float *q, const float *prefix_k, const float *generated_k, const float *v,

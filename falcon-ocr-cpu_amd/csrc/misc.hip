@@ -160,14 +160,24 @@ __global__ __launch_bounds__(256) void row_scales_fixed_kernel(const float *__re
 }
 
 // argmax (src/runner/mod.rs:916-930): first index of the maximum, and a flag
-// when any value is non-finite. One workgroup of 1024 threads per row; each
-// thread keeps the first maximum of its own values (visited in ascending
-// index order), and the workgroup combines (value, index) pairs, the smaller
-// index winning ties. Every thread issues its loads of a pass (8 float4, or 8
-// floats for rows that are not 16-byte aligned) before comparing them.
-__global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ logits, int vocab,
-                                                      uint32_t *__restrict__ result) {
-  const float *row = logits + static_cast<size_t>(blockIdx.x) * vocab;
+// when any value is non-finite. A row is cut into `parts` runs of `chunk`
+// values (a multiple of 4), one workgroup each; each thread keeps the first
+// maximum of its own values (visited in ascending index order), the workgroup
+// combines (value, index) pairs, the smaller index winning ties, and writes
+// its part's straight into pinned host memory, where the host, which waits for
+// the call anyway, takes the first largest of the parts. Every thread issues
+// its loads of a pass (4 float4, or 4 floats for rows that are not 16-byte
+// aligned) before comparing them.
+// Bound: latency. One workgroup per row read 65,536 logits in 9.4 us, and the
+// result's copy through pageable memory took the host about 11 us more than
+// waiting for the kernel.
+__global__ __launch_bounds__(256) void argmax_kernel(const float *__restrict__ logits, int vocab, int parts, int chunk,
+                                                     ArgmaxPart *__restrict__ result) {
+  const int part = blockIdx.x % parts;
+  const float *row = logits + static_cast<size_t>(blockIdx.x / parts) * vocab;
+  const long begin = static_cast<long>(part) * chunk;
+  const int first = static_cast<int>(begin < vocab ? begin : vocab);
+  const int end = static_cast<int>(begin + chunk < vocab ? begin + chunk : vocab);
   const int tid = threadIdx.x;
   float best = -__builtin_inff();
   int best_i = -1;
@@ -181,39 +191,35 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
   };
   const bool vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
   if (vec) {
-    const int quads = vocab / 4;
-    for (int base = 0; base < quads; base += 8 * 1024) {
-      float4 q[8];
+    const int quads = (end - first) / 4;
+    const float4 *src = reinterpret_cast<const float4 *>(row + first);
+    for (int base = 0; base < quads; base += 4 * 256) {
+      float4 q[4];
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const int at = base + 1024 * j + tid;
-        q[j] = at < quads ? reinterpret_cast<const float4 *>(row)[at] : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int j = 0; j < 4; j++) {
+        const int at = base + 256 * j + tid;
+        q[j] = at < quads ? src[at] : make_float4(0.f, 0.f, 0.f, 0.f);
       }
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const int at = base + 1024 * j + tid;
+      for (int j = 0; j < 4; j++) {
+        const int at = base + 256 * j + tid;
         if (at < quads) {
-          visit(q[j].x, 4 * at);
-          visit(q[j].y, 4 * at + 1);
-          visit(q[j].z, 4 * at + 2);
-          visit(q[j].w, 4 * at + 3);
+          visit(q[j].x, first + 4 * at);
+          visit(q[j].y, first + 4 * at + 1);
+          visit(q[j].z, first + 4 * at + 2);
+          visit(q[j].w, first + 4 * at + 3);
         }
       }
     }
-    for (int i = 4 * quads + tid; i < vocab; i += 1024) visit(row[i], i);
+    for (int i = first + 4 * quads + tid; i < end; i += 256) visit(row[i], i);
   } else {
-    for (int base = 0; base < vocab; base += 8 * 1024) {
-      float v[8];
+    for (int base = first; base < end; base += 4 * 256) {
+      float v[4];
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const int at = base + 1024 * j + tid;
-        v[j] = at < vocab ? row[at] : 0.0f;
-      }
+      for (int j = 0; j < 4; j++) v[j] = end - base > 256 * j + tid ? row[base + 256 * j + tid] : 0.0f;
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const int at = base + 1024 * j + tid;
-        if (at < vocab) visit(v[j], at);
-      }
+      for (int j = 0; j < 4; j++)
+        if (end - base > 256 * j + tid) visit(v[j], base + 256 * j + tid);
     }
   }
   // Wave, then workgroup combination.
@@ -227,9 +233,9 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
     }
     nonfinite |= __shfl_xor(nonfinite, off);
   }
-  __shared__ float s_val[16];
-  __shared__ int s_idx[16];
-  __shared__ int s_bad[16];
+  __shared__ float s_val[4];
+  __shared__ int s_idx[4];
+  __shared__ int s_bad[4];
   if ((tid & 63) == 0) {
     s_val[tid >> 6] = best;
     s_idx[tid >> 6] = best_i;
@@ -239,15 +245,15 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
   if (tid == 0) {
     float fv = s_val[0];
     int fi = s_idx[0], bad = s_bad[0];
-    for (int w = 1; w < 16; w++) {
+    for (int w = 1; w < 4; w++) {
       bad |= s_bad[w];
       if (s_idx[w] >= 0 && (fi < 0 || s_val[w] > fv || (s_val[w] == fv && s_idx[w] < fi))) {
         fv = s_val[w];
         fi = s_idx[w];
       }
     }
-    result[2 * blockIdx.x] = static_cast<uint32_t>(fi);
-    result[2 * blockIdx.x + 1] = static_cast<uint32_t>(bad);
+    *reinterpret_cast<uint4 *>(result + blockIdx.x) =
+        make_uint4(__float_as_uint(fv), static_cast<uint32_t>(fi), static_cast<uint32_t>(bad), 0);
   }
 }
 
@@ -312,10 +318,10 @@ int launch_row_scales(Ctx *ctx, const float *h, size_t rows, size_t width, float
   return FOCR_OK;
 }
 
-int launch_argmax(Ctx *ctx, const float *logits, size_t rows, size_t vocab, uint32_t *result_dev) {
-  FOCR_REQUIRE(rows < (size_t(1) << 31), FOCR_E_SHAPE, "focr_argmax: too many rows");
-  hipLaunchKernelGGL(argmax_kernel, dim3(static_cast<unsigned>(rows)), dim3(1024), 0, ctx->stream, logits,
-                     static_cast<int>(vocab), result_dev);
+int launch_argmax(Ctx *ctx, const float *logits, size_t rows, size_t vocab, int parts, int chunk, ArgmaxPart *result) {
+  FOCR_REQUIRE(rows * parts < (size_t(1) << 31), FOCR_E_SHAPE, "focr_argmax: too many rows");
+  hipLaunchKernelGGL(argmax_kernel, dim3(static_cast<unsigned>(rows * parts)), dim3(256), 0, ctx->stream, logits,
+                     static_cast<int>(vocab), parts, chunk, result);
   FOCR_HIP_CHECK(hipGetLastError());
   return FOCR_OK;
 }

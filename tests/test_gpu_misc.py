@@ -87,6 +87,23 @@ def test_argmax_unaligned_rows_and_ties(fh):
     assert fh.argmax(to_dev(big), 2, 70001) == [oracle.argmax(r) for r in big]
 
 
+@pytest.mark.parametrize("rows,vocab", [(1, 4096), (1, 4097), (2, 65536), (3, 8195), (1, 300001), (700, 12289)])
+def test_argmax_parts(fh, rows, vocab):
+    # A row is cut into up to 64 parts of at least 4,096 logits (fewer parts
+    # with many rows): ties across the parts' borders, the ragged last part, a
+    # non-finite value in any part.
+    parts = min(64, max(1, 1024 // rows), -(-vocab // 4096))
+    chunk = -(-(-(-vocab // parts)) // 4) * 4
+    logits = gen.normal((rows, vocab), 1.0, 36)
+    logits[0, vocab - 1] = np.float32(9.0)
+    if rows > 1:
+        logits[1, min(chunk, vocab - 1)] = logits[1, min(chunk, vocab - 1) - 1] = np.float32(9.0)
+    assert fh.argmax(to_dev(logits), rows, vocab) == [int(np.argmax(r)) for r in logits]
+    logits[rows - 1, vocab - 2] = np.nan
+    with pytest.raises(fh.FocrError, match="nonfinite"):
+        fh.argmax(to_dev(logits), rows, vocab)
+
+
 def test_argmax_ties_across_partial_workgroups(fh):
     # Rows are split into 2,048-logit partials combined per row: a tie across
     # a partial boundary, across distant partials and inside one, a maximum in
