@@ -30,6 +30,17 @@ constexpr long long kSplitItemsF32 = 3072;
 constexpr long long kSplitItemsBf16 = 1536;
 constexpr long long kSplitItemsPair = 3072;
 constexpr long long kMinChunkKeys = 1024;
+// With at most one workgroup per compute unit (tiles x heads), the FP32 and
+// FP16-pair kernels are bound by the chain of one workgroup's key tiles (1.35
+// us each with one wave per SIMD): such calls take parts of down to 192 keys,
+// about two workgroups per compute unit. FP16-pair prefill, 16 heads, us: 225
+// rows 27.7 -> 25.8, 400 34 -> 29, 700 48 -> 36, 1,000 64 -> 42, 1,501 66 ->
+// 55, 2,000 77 -> 75; at 2,500 rows (320 workgroups) 96 -> 102, and at 144
+// rows two parts and their merge 22.4 -> 24.3, so neither is split further.
+// (The BF16 kernel's tiles are too short for it: 1,000 rows 26.7 -> 25.0, 400
+// rows 15.2 -> 15.6.)
+constexpr int kSmallGrid = 256;
+constexpr long long kSmallItems = 512, kSmallChunkKeys = 192;
 
 // Work plan (computed on the host, passed by value): query tiles in dispatch
 // order i (tile tiles - 1 - i: the latest, longest tiles first), each split
@@ -61,7 +72,7 @@ __host__ __device__ inline int tile_visible_end(int tile, int query_len, int que
 // Builds the plan for `tiles` (<= kMaxTiles) tiles; part sizes are multiples
 // of `align` keys. Returns the number of work items; *slots = partial slots.
 inline int make_plan(Plan &plan, int tiles, int query_len, int query_offset, int image_start, int image_end,
-                     int n_heads, int align, long long target_items, int *slots_out) {
+                     int n_heads, int align, long long target_items, bool small_grid, int *slots_out) {
   long long total = 0;
   int vis[kMaxTiles], most = 0;
   for (int t = 0; t < tiles; t++) {
@@ -74,6 +85,11 @@ inline int make_plan(Plan &plan, int tiles, int query_len, int query_offset, int
   // Tiles of nearly equal cost (an all-image or short prefill) balance by
   // themselves: splitting them would only add the merge traffic.
   if (5LL * most <= 6LL * total / (tiles > 0 ? tiles : 1)) chunk = most;
+  if (small_grid && static_cast<long long>(tiles) * n_heads <= kSmallGrid) {
+    const long long few = total * static_cast<long long>(n_heads) / kSmallItems;
+    const long long small = ((few > kSmallChunkKeys ? few : kSmallChunkKeys) + align - 1) / align * align;
+    chunk = small < chunk ? small : chunk;
+  }
   int items = 0, slots = 0;
   for (int i = 0; i < tiles; i++) {
     const int end = vis[tiles - 1 - i];

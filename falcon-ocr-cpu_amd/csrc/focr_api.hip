@@ -42,6 +42,12 @@ int ensure_scratch(Ctx *ctx, size_t bytes) {
   return FOCR_OK;
 }
 
+bool scratch_fits(Ctx *ctx, size_t bytes) {
+  if (bytes <= ctx->scratch_bytes) return true;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+}
+
 // The context's work moves to a new stream only behind everything already
 // queued on the old one (an event the new stream waits for), so a call on the
 // new stream cannot overwrite the context scratch while an earlier call on

@@ -55,6 +55,9 @@ struct Ctx {
 
 // Grows the context scratch to at least `bytes` (hipMalloc on growth only).
 int ensure_scratch(Ctx *ctx, size_t bytes);
+// Whether ensure_scratch(ctx, bytes) can succeed now: it cannot grow while the
+// stream is being captured.
+bool scratch_fits(Ctx *ctx, size_t bytes);
 // Resolves the device address of the no-alloc decode scratch for `device`
 // (which must be current); once per device.
 int noalloc_scratch_init(int device);

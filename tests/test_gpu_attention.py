@@ -135,6 +135,42 @@ def test_split_key_ranges_full_compare(fh, static, exp):
     close(got, want)
 
 
+def norm8(n_heads, rows, seed):
+    x = gen.normal((rows, n_heads, 64), 1.0, seed)
+    return (x * (8.0 / np.linalg.norm(x, axis=-1, keepdims=True))).astype(np.float32)
+
+
+# Small grids split their tiles' keys into parts of down to 192 keys: around
+# the first split, where the last tile is one row, the last small grid (2,048
+# rows of 16 heads) and the first that is not one.
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("products", ["split", "fp32"])
+@pytest.mark.parametrize("L,image", [(192, (0, 100)), (193, (0, 193)), (385, (3, 200)), (1030, (0, 600)), (2048, (0, 1300)),
+                                     (2049, (0, 1300))])
+def test_small_grids_split_their_keys(fh, L, image, products, static):
+    oracle.set_threads(8)
+    q, k, v = norm8(16, L, 401).reshape(-1), norm8(16, L, 402).reshape(-1), gen.normal(L * 8 * 64, 1.0, 403)
+    sinks = gen.uniform(16, -2.0, 2.0, 404)
+    opts = fh.PrefillOptions(fp32_softmax=fh.Softmax.STATIC if static else fh.Softmax.ONLINE,
+                             split_products=products == "split")
+    got = run(fh, q, k, v, sinks, L, (0, *image), opts)
+    want = oracle.attention_prefill(q, k, v, L, L, L, 16, 8, 0, *image, sinks, static=static)
+    close(got, want)
+
+
+def test_few_rows_over_a_long_cache_split_its_keys(fh):
+    # Nine query rows behind 4,000 prefix keys: one tile, split by keys.
+    oracle.set_threads(8)
+    rows, prefix = 9, 4000
+    total = prefix + rows
+    q, k = norm8(16, rows, 411).reshape(-1), norm8(16, prefix, 412).reshape(-1)
+    gk, v = norm8(8, rows, 413).reshape(-1), gen.normal(total * 8 * 64, 1.0, 414)
+    sinks = gen.uniform(16, -2.0, 2.0, 415)
+    got = run(fh, q, k, v, sinks, rows, (prefix, 0, 2500), fh.PrefillOptions(), prefix=prefix, total=total, generated=gk)
+    want = oracle.attention_prefill(q, k, v, rows, prefix, total, 16, 8, prefix, 0, 2500, sinks, generated_k=gk)
+    close(got, want)
+
+
 def test_config5_prefill_whole(fh):
     # BASELINE config 5's prefill attention: 16,320 rows, image [0, 4096),
     # split key ranges; every output.
