@@ -21,12 +21,11 @@
 // single short kernel.
 //
 // Decode: one workgroup task per (group, key chunk) serves both heads of the
-// pair (the record is read once for both); its four waves take interleaved
-// 16-key iterations with the compact decode kernel's lane map (lane group
-// lg = lane / 16 takes keys 4i + lg, lane lp = lane % 16 dims 4lp..4lp+3),
-// every lane reading its codes at offsets selected without branches. Online
-// softmax per (head, row), the four waves merged in a fixed order through
-// LDS, then the shared combine kernel. With the cache's fast exp
+// pair (the record is read once for both) and up to three query rows; its four
+// waves take interleaved 16-key slices (split_scan_kernel's lane map), every
+// lane reading its codes at offsets selected without branches. Online softmax
+// per (head, row), the four waves merged in a fixed order through LDS, then
+// the shared combine kernel. With the cache's fast exp
 // (SplitPrefix::with_fast_exp, kv.rs:423; the polynomial exp of the
 // reference's exp_shifted, decode.rs:346-347) the per-key probabilities
 // p = exp(s - max) use the hardware exp2 of log2(e) * x instead of the device
@@ -83,8 +82,6 @@ float *noalloc_scratch(int device) {
 }
 }  // namespace
 
-inline const hipStream_t kNoStream = reinterpret_cast<hipStream_t>(~uintptr_t(0));
-
 struct KvSplit {
   int bits = 8;
   int n_heads = 0, n_kv = 0;
@@ -94,13 +91,10 @@ struct KvSplit {
   unsigned char *tail = nullptr;     // [n_kv][capacity - prefix_len][tail_bytes]
   size_t records_alloc = 0, tail_alloc = 0;  // bytes allocated, at least what the current sizes need
   size_t device_bytes = 0;
-  // The first stream that used this cache since it was sealed (kNoStream:
-  // none), and whether there is work on it that this stream does not order
-  // (another stream's, or a capture's, which may be replayed anywhere): what
-  // focr_kv_reseal has to wait for. Atomic: contexts may read one cache from
-  // several threads.
-  std::atomic<hipStream_t> stream{kNoStream};
-  std::atomic<bool> spread{false};
+  // Whether any call has queued work on the records since they were sealed
+  // (the seal itself is synchronous): focr_kv_reseal then waits for the device.
+  // Atomic: contexts may read one cache from several threads.
+  mutable std::atomic<bool> used{false};
   bool fast_exp = false;  // SplitPrefix::fast_exp (kv.rs:168-170)
 };
 
@@ -403,68 +397,19 @@ __device__ __forceinline__ float4 codes4(const unsigned char *p) {
 
 __device__ __forceinline__ float4 scale4(float4 c, float s) { return make_float4(c.x * s, c.y * s, c.z * s, c.w * s); }
 
-// A key's (both heads') and value's decoded values for lane lp (dims
-// 4lp..4lp+3 of each 64-wide head). Branch-free over the record kind: in a
-// prefix record head 2g's key is codes [0, 64) (T then S(2g)) and head
-// 2g+1's is T then S(2g+1) = codes [64, 96); a tail record holds one key
-// [0, 64) for both heads. The BF16 steps follow the codes, 16-byte aligned.
-struct KeyVal {
-  float4 k0, k1, v;
-};
-
-__device__ __forceinline__ float step_of(uint4 w, int i) {
-  const uint32_t word = i < 2 ? w.x : i < 4 ? w.y : i < 6 ? w.z : w.w;
-  return bf16_widen(static_cast<uint16_t>((i & 1) ? word >> 16 : word & 0xffffu));
-}
-
-template <typename C>
-__device__ __forceinline__ KeyVal load_key(const SplitDecArgs &a, int g, int j, int lp) {
-  const bool prefix = j < a.prefix_len;
-  const unsigned char *rec =
-      prefix ? a.records + (static_cast<size_t>(g) * a.prefix_len + j) * a.record_bytes
-             : a.tail + (static_cast<size_t>(g) * a.tail_capacity + (j - a.prefix_len)) * a.tail_bytes;
-  const int hi = lp >> 3;
-  const int k1_at = prefix ? 4 * lp + 32 * hi : 4 * lp;
-  const int v_at = (prefix ? 96 : 64) + 4 * lp;
-  const uint4 steps = *reinterpret_cast<const uint4 *>(rec + (prefix ? kRecord : kTail) * sizeof(C));
-  const float4 c0 = codes4<C>(rec + 4 * lp * sizeof(C));
-  const float4 c1 = codes4<C>(rec + k1_at * sizeof(C));
-  const float4 cv = codes4<C>(rec + v_at * sizeof(C));
-  KeyVal kv;
-  kv.k0 = scale4(c0, step_of(steps, hi));
-  kv.k1 = scale4(c1, step_of(steps, prefix ? 2 * hi : hi));
-  kv.v = scale4(cv, step_of(steps, (prefix ? 3 : 2) + hi));
-  return kv;
-}
-
-// load_key of a prefix record that sits in LDS at `rec`.
-template <typename C>
-__device__ __forceinline__ KeyVal lds_key(const unsigned char *rec, int lp) {
-  const int hi = lp >> 3;
-  const uint4 steps = *reinterpret_cast<const uint4 *>(rec + kRecord * sizeof(C));
-  const float4 c0 = codes4<C>(rec + 4 * lp * sizeof(C));
-  const float4 c1 = codes4<C>(rec + (4 * lp + 32 * hi) * sizeof(C));
-  const float4 cv = codes4<C>(rec + (96 + 4 * lp) * sizeof(C));
-  KeyVal kv;
-  kv.k0 = scale4(c0, step_of(steps, hi));
-  kv.k1 = scale4(c1, step_of(steps, 2 * hi));
-  kv.v = scale4(cv, step_of(steps, 3 + hi));
-  return kv;
-}
-
 constexpr int kKpl = 4;  // keys per lane group per iteration (16 per wave)
 constexpr int kRoundKeys = 16 * kWaves;  // positions per workgroup round
 
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void global_void;
 
-// M: query rows. One workgroup per task (group g, key chunk c) serves heads
-// 2g and 2g + 1 in rounds of 64 positions: wave w takes positions 16w ..
-// 16w + 15 of each round, and the four waves' states are merged in a fixed
-// order through LDS. The round's prefix records (contiguous in HBM) are
-// copied to LDS by the LDS-DMA path, 16 bytes per lane, the next round's
-// while the current one is scored; generated keys (the tail) and the padding
-// keys past the last visible one are read from HBM as before.
+// One workgroup per task (group g, key chunk c) serves heads 2g and 2g + 1 in
+// rounds of 64 positions: wave w takes positions 16w .. 16w + 15 of each
+// round, and the four waves' states are merged in a fixed order through LDS.
+// The round's prefix records (contiguous in HBM) are copied to LDS by the
+// LDS-DMA path, 16 bytes per lane, the next round's while the current one is
+// scored; generated keys (the tail) and the padding keys past the last
+// visible one are read from HBM.
 template <typename C>
 struct RoundBuf {
   static constexpr int kCopies = (kRoundKeys * (kRecord * static_cast<int>(sizeof(C)) + 16) + 4095) / 4096;
@@ -483,178 +428,6 @@ __device__ __forceinline__ float prob_exp(float x) {
     return expf_acc(x);
 }
 
-template <typename C, int M, bool FAST>
-__global__ __launch_bounds__(256) void split_partial_kernel(SplitDecArgs a, int iters, int rows) {
-  __shared__ float4 s_o[kWaves][2][M][16];
-  __shared__ float2 s_md[kWaves][2][M];
-  // Two distinct LDS objects, so the compiler sees that reading one does not
-  // wait for the copies into the other.
-  __shared__ RoundBuf<C> rb0, rb1;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int lg = lane >> 4, lp = lane & 15;
-  const int task = blockIdx.x;
-  const int c = task % a.chunks, g = task / a.chunks;
-  const int key0 = c * iters * 4 * kKpl;
-  int vis[M], limit = 0;
-#pragma unroll
-  for (int r = 0; r < M; r++) {
-    vis[r] = a.last - rows + r + 1;
-    limit = vis[r] > limit ? vis[r] : limit;
-  }
-  float4 qv[2][M];
-#pragma unroll
-  for (int e = 0; e < 2; e++)
-#pragma unroll
-    for (int r = 0; r < M; r++)
-      qv[e][r] = ld4(a.q + (static_cast<size_t>(r) * a.n_heads + 2 * g + e) * 64 + 4 * lp);
-  const float ninf = -__builtin_inff();
-  float m[2][M], den[2][M];
-  float4 o[2][M];
-#pragma unroll
-  for (int e = 0; e < 2; e++)
-#pragma unroll
-    for (int r = 0; r < M; r++) {
-      m[e][r] = ninf;
-      den[e][r] = 0.0f;
-      o[e][r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-  // Round t's copies: chunk q = tid + 256 i of the rows [b, b + 64) of group
-  // g's prefix records (b = key0 + 64 t); chunks past the prefix (or a round
-  // entirely in the tail) copy the group's first chunk instead, into slots
-  // that are never read.
-  constexpr int kCopies = RoundBuf<C>::kCopies;
-  const int rbytes = a.record_bytes;
-  const unsigned char *group_base = a.records + static_cast<size_t>(g) * a.prefix_len * rbytes;
-  auto issue = [&](RoundBuf<C> &dst, int t) {
-    const int b = key0 + kRoundKeys * t;
-    const int in_prefix = a.prefix_len - b;
-    const int valid = in_prefix <= 0 ? 0 : (in_prefix < kRoundKeys ? in_prefix : kRoundKeys) * rbytes;
-    const unsigned char *src = group_base + static_cast<size_t>(in_prefix > 0 ? b : 0) * rbytes;
-#pragma unroll
-    for (int i = 0; i < kCopies; i++) {
-      const int off = (threadIdx.x + 256 * i) * 16;
-      __builtin_amdgcn_global_load_lds((global_void *)(src + (off < valid ? off : 0)),
-                                       (lds_void *)(&dst.chunk[64 * wave + 256 * i]), 16, 0, 0);
-    }
-  };
-  auto load = [&](KeyVal (&kb)[kKpl], int it) {
-#pragma unroll
-    for (int i = 0; i < kKpl; i++) {
-      const int j = key0 + 16 * it + 4 * i + lg;
-      kb[i] = load_key<C>(a, g, j < limit ? j : 0, lp);
-    }
-  };
-  auto consume = [&](const KeyVal (&kb)[kKpl], int it) {
-    float s[2][kKpl][M];
-#pragma unroll
-    for (int i = 0; i < kKpl; i++) {
-      const int j = key0 + 16 * it + 4 * i + lg;
-#pragma unroll
-      for (int e = 0; e < 2; e++) {
-        const float4 k = e == 0 ? kb[i].k0 : kb[i].k1;
-#pragma unroll
-        for (int r = 0; r < M; r++) {
-          float d = qv[e][r].x * k.x;
-          d = fmaf_(qv[e][r].y, k.y, d);
-          d = fmaf_(qv[e][r].z, k.z, d);
-          d = fmaf_(qv[e][r].w, k.w, d);
-          d = row_sum16(d) * 0.125f;
-          s[e][i][r] = j < vis[r] ? d : ninf;
-        }
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 2; e++)
-#pragma unroll
-      for (int r = 0; r < M; r++) {
-        float bmax = s[e][0][r];
-#pragma unroll
-        for (int i = 1; i < kKpl; i++) bmax = s[e][i][r] > bmax ? s[e][i][r] : bmax;
-        const float mn = bmax > m[e][r] ? bmax : m[e][r];
-        if (mn == ninf) continue;
-        const float rs = m[e][r] == ninf ? 0.0f : expf_acc(m[e][r] - mn);
-        den[e][r] = den[e][r] * rs;
-        o[e][r] = scale4(o[e][r], rs);
-        m[e][r] = mn;
-#pragma unroll
-        for (int i = 0; i < kKpl; i++) {
-          const float p = s[e][i][r] == ninf ? 0.0f : prob_exp<FAST>(s[e][i][r] - mn);
-          const float4 v = kb[i].v;
-          den[e][r] = den[e][r] + p;
-          o[e][r] = make_float4(fmaf_(p, v.x, o[e][r].x), fmaf_(p, v.y, o[e][r].y), fmaf_(p, v.z, o[e][r].z),
-                                fmaf_(p, v.w, o[e][r].w));
-        }
-      }
-  };
-  // iters is a multiple of kWaves: every wave takes iters / kWaves
-  // iterations, one per round. Past the last round the copy repeats it into
-  // the free buffer (no branch around the copies: a branch join would make
-  // the compiler wait for every copy in flight).
-  const int rounds = iters / kWaves;
-  auto round = [&](const RoundBuf<C> &cur, RoundBuf<C> &next, int t) __attribute__((always_inline)) {
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's copies of round t
-    __syncthreads();                     // everyone's copies; nobody still reads `next`
-    issue(next, t + 1 < rounds ? t + 1 : rounds - 1);
-    const int it = kWaves * t + wave, b = key0 + kRoundKeys * t;
-    KeyVal kb[kKpl];
-    // A round wholly inside the visible prefix is scored from LDS; the
-    // round that reaches the tail or the last visible key reads HBM. Each
-    // branch consumes its own keys: a key loaded from HBM must not reach
-    // past the join, where waiting for it would also wait for the copies.
-    if (b + kRoundKeys <= a.prefix_len && b + kRoundKeys <= limit) {
-#pragma unroll
-      for (int i = 0; i < kKpl; i++)
-        kb[i] = lds_key<C>(reinterpret_cast<const unsigned char *>(cur.chunk) + (16 * wave + 4 * i + lg) * rbytes, lp);
-      consume(kb, it);
-    } else {
-      load(kb, it);
-      consume(kb, it);
-    }
-  };
-  issue(rb0, 0);
-  int t = 0;
-  for (; t + 2 <= rounds; t += 2) {
-    round(rb0, rb1, t);
-    round(rb1, rb0, t + 1);
-  }
-  if (t < rounds) round(rb0, rb1, t);
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // the repeated copies land before LDS is reused
-#pragma unroll
-  for (int e = 0; e < 2; e++)
-#pragma unroll
-    for (int r = 0; r < M; r++) {
-#pragma unroll
-      for (int mask = 16; mask <= 32; mask *= 2) {
-        const float m2 = xor_lane(m[e][r], mask), d2 = xor_lane(den[e][r], mask);
-        const float4 o2 = make_float4(xor_lane(o[e][r].x, mask), xor_lane(o[e][r].y, mask),
-                                      xor_lane(o[e][r].z, mask), xor_lane(o[e][r].w, mask));
-        merge(m[e][r], den[e][r], o[e][r], m2, d2, o2);
-      }
-      if (lg == 0) s_o[wave][e][r][lp] = o[e][r];
-      if (lane == 0) s_md[wave][e][r] = make_float2(m[e][r], den[e][r]);
-    }
-  __syncthreads();
-  // Wave w's lanes 16e' + lp merge the four waves for (head e, rows r = w,
-  // w + 4): lane group lg < 2 is the head.
-  if (lg < 2) {
-    const int e = lg;
-#pragma unroll
-    for (int r = 0; r < M; r++) {
-      if (r % kWaves != wave) continue;
-      float2 md = s_md[0][e][r];
-      float4 acc = s_o[0][e][r][lp];
-#pragma unroll
-      for (int w = 1; w < kWaves; w++) {
-        const float2 md2 = s_md[w][e][r];
-        merge(md.x, md.y, acc, md2.x, md2.y, s_o[w][e][r][lp]);
-      }
-      const size_t slot = (static_cast<size_t>(r) * a.n_heads + 2 * g + e) * a.chunks + c;
-      *reinterpret_cast<float4 *>(a.part_o + slot * 64 + 4 * lp) = acc;
-      if (lp == 0) *reinterpret_cast<float2 *>(a.part_md + slot * 2) = md;
-    }
-  }
-}
-
 // Code I (0..3) of a 32-bit word of four Q8 codes, or (0..1) of two Q16
 // codes, as a float (exact). Plain C: the compiler forms the SDWA conversion
 // itself and, unlike for inline assembly, knows it needs no wait state
@@ -667,8 +440,8 @@ __device__ __forceinline__ float word_code(uint32_t w) {
     return static_cast<float>(static_cast<int16_t>(w >> (16 * I)));
 }
 
-// The scan for one or two query rows, with the work of a 16-key slice laid
-// out so that no lane repeats another's: for the scores, lane (key kk, head
+// The scan of M query rows (rows M y .. of the call for grid row y), with the
+// work of a 16-key slice laid out so that no lane repeats another's: for the scores, lane (key kk, head
 // e, half) forms the dot of its 32 dims of head 2g + e with the key's codes
 // (T for half 0, S(2g + e) for half 1 of a prefix record; the key's dims
 // 0-31 / 32-63 of a tail record), scaled once by the block's step, and the
@@ -698,13 +471,14 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kk = lane & 15, e = (lane >> 4) & 1, half = lane >> 5;
   const int dq = lane & 15, ks = lane >> 4;
-  const int task = blockIdx.x;
+  const int task = blockIdx.x, row0 = M * blockIdx.y;
   const int c = task % a.chunks, g = task / a.chunks;
   const int key0 = c * iters * 4 * kKpl;
   int vis[M], limit = 0;
 #pragma unroll
   for (int r = 0; r < M; r++) {
-    vis[r] = a.last - rows + r + 1;
+    const int row = row0 + r < rows ? row0 + r : rows - 1;  // past the last row: it again, not written
+    vis[r] = a.last - rows + row + 1;
     limit = vis[r] > limit ? vis[r] : limit;
   }
   constexpr int kCopies = RoundBuf<C>::kCopies;
@@ -752,7 +526,8 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
     for (int r = 0; r < M; r++)
 #pragma unroll
       for (int i = 0; i < 8; i++) {
-        const float4 t = ld4(a.q + (static_cast<size_t>(r) * a.n_heads + 2 * g + e) * 64 + 32 * half + 4 * i);
+        const int row = row0 + r < rows ? row0 + r : rows - 1;
+        const float4 t = ld4(a.q + (static_cast<size_t>(row) * a.n_heads + 2 * g + e) * 64 + 32 * half + 4 * i);
         qv[r][4 * i] = t.x;
         qv[r][4 * i + 1] = t.y;
         qv[r][4 * i + 2] = t.z;
@@ -870,8 +645,9 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
     issue(next, t + 1 < rounds ? t + 1 : rounds - 1);
     const int b = key0 + kRoundKeys * t;
     const int bw = b + 16 * wave;
-    // As in split_partial_kernel: a round wholly inside the visible prefix is
-    // scored from LDS, the others read HBM, each branch consuming its own keys.
+    // A round wholly inside the visible prefix is scored from LDS, the others
+    // (generated keys, padding past the last visible one) read HBM, each branch
+    // consuming its own keys so that no wait at the join covers the copies.
     if (b + kRoundKeys <= a.prefix_len && b + kRoundKeys <= limit) {
       const unsigned char *base = reinterpret_cast<const unsigned char *>(cur.chunk) + 16 * wave * rbytes;
       slice(bw, [&](int q) { return RecRef{base + q * rbytes, true}; });
@@ -921,7 +697,7 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
     const int he = lg;
 #pragma unroll
     for (int r = 0; r < M; r++) {
-      if (r % kWaves != wave) continue;
+      if (r % kWaves != wave || row0 + r >= rows) continue;
       float2 md = s_md[0][he][r];
       float4 accv = s_o[0][he][r][lp];
 #pragma unroll
@@ -929,7 +705,7 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
         const float2 md2 = s_md[w][he][r];
         merge(md.x, md.y, accv, md2.x, md2.y, s_o[w][he][r][lp]);
       }
-      const size_t slot = (static_cast<size_t>(r) * a.n_heads + 2 * g + he) * a.chunks + c;
+      const size_t slot = (static_cast<size_t>(row0 + r) * a.n_heads + 2 * g + he) * a.chunks + c;
       *reinterpret_cast<float4 *>(a.part_o + slot * 64 + 4 * lp) = accv;
       if (lp == 0) *reinterpret_cast<float2 *>(a.part_md + slot * 2) = md;
     }
@@ -938,7 +714,7 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
 
 // `fixed` (optional): a caller-provided partial-state buffer of
 // `fixed_bytes` used instead of the context scratch (nothing is allocated).
-template <typename C, int M, bool ROW = false>
+template <typename C, int G, bool ROW = false>
 int launch_split(Ctx *ctx, SplitDecArgs a, int rows, bool fast, const float *sinks, float *out, float *fixed,
                  size_t fixed_bytes) {
   // Keys per workgroup task, whole multiples of 64 keys (every wave of the
@@ -951,8 +727,18 @@ int launch_split(Ctx *ctx, SplitDecArgs a, int rows, bool fast, const float *sin
   // against 17.0 with 1,024; 65,536 positions 28.1 us with 1,024 tasks
   // against 29.0 with 512; 4,160 positions 12.8 us with 520 tasks against
   // 13.2 with 264.
-  const long limit = a.last;
-  long per = limit <= 32768 ? (limit * a.n_kv / 512 + 32) / 64 * 64 : ((limit * a.n_kv + 1023) / 1024 + 63) / 64 * 64;
+  // More than two rows run in groups of G rows per workgroup (grid y), each
+  // scanning the records on its own: the records come from L2 after the first
+  // group, and the lane map that repeats no lane's work outweighs reading them
+  // again. Three rows to a group where that makes fewer groups (four rows: two
+  // of two); with several groups, about 256 tasks each. Q16 records, 200 /
+  // 4,000 / 6,544 / 16,320 positions, us with the combine, before (one
+  // workgroup for all rows, 16 lanes per key) -> now: 3 rows 11.5 / 15.2 / 19.1 /
+  // 29.5 -> 8.7 / 11.5 / 13.8 / 19.9, 5 rows 15.4 / 21.2 / 26.8 / 41.3 -> 9.1 /
+  // 14.4 / 21.7 / 27.6 (groups of two 7.9 / 16.3 / 21.0 / 31.6), 8 rows 21.1 /
+  // 40.5 / 55.4 / 84.1 -> 8.7 / 19.0 / 25.3 / 39.7.
+  const long limit = a.last, target = rows <= G ? 512 : 256;
+  long per = limit <= 32768 ? (limit * a.n_kv / target + 32) / 64 * 64 : ((limit * a.n_kv + 1023) / 1024 + 63) / 64 * 64;
   const long min_per = ((limit + kMaxChunks - 1) / kMaxChunks + 63) / 64 * 64;
   if (per < min_per) per = min_per;
   if (per < 64) per = 64;
@@ -972,22 +758,11 @@ int launch_split(Ctx *ctx, SplitDecArgs a, int rows, bool fast, const float *sin
     a.part_o = static_cast<float *>(ctx->scratch);
   }
   a.part_md = a.part_o + slots * 64;
-  if constexpr (M <= 2) {
-    if (fast)
-      hipLaunchKernelGGL((split_scan_kernel<C, M, true, ROW>), dim3(a.tasks), dim3(64 * kWaves), 0, ctx->stream, a,
-                         iters, rows);
-    else
-      hipLaunchKernelGGL((split_scan_kernel<C, M, false, ROW>), dim3(a.tasks), dim3(64 * kWaves), 0, ctx->stream, a,
-                         iters, rows);
-  } else {
-    static_assert(!ROW, "the fused row step takes one row");
-    if (fast)
-      hipLaunchKernelGGL((split_partial_kernel<C, M, true>), dim3(a.tasks), dim3(64 * kWaves), 0, ctx->stream, a,
-                         iters, rows);
-    else
-      hipLaunchKernelGGL((split_partial_kernel<C, M, false>), dim3(a.tasks), dim3(64 * kWaves), 0, ctx->stream, a,
-                         iters, rows);
-  }
+  const dim3 grid(static_cast<unsigned>(a.tasks), static_cast<unsigned>((rows + G - 1) / G));
+  if (fast)
+    hipLaunchKernelGGL((split_scan_kernel<C, G, true, ROW>), grid, dim3(64 * kWaves), 0, ctx->stream, a, iters, rows);
+  else
+    hipLaunchKernelGGL((split_scan_kernel<C, G, false, ROW>), grid, dim3(64 * kWaves), 0, ctx->stream, a, iters, rows);
   FOCR_HIP_CHECK(hipGetLastError());
   CombineArgs cb;
   cb.part_o = a.part_o;
@@ -1007,13 +782,9 @@ int launch_split_rows(Ctx *ctx, const SplitDecArgs &a, int rows, bool fast, cons
                       float *fixed, size_t fixed_bytes) {
   switch (rows) {
     case 1: return launch_split<C, 1>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
-    case 2: return launch_split<C, 2>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
-    case 3: return launch_split<C, 3>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
-    case 4: return launch_split<C, 4>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
-    case 5: return launch_split<C, 5>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
-    case 6: return launch_split<C, 6>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
-    case 7: return launch_split<C, 7>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
-    default: return launch_split<C, 8>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
+    case 2:
+    case 4: return launch_split<C, 2>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
+    default: return launch_split<C, 3>(ctx, a, rows, fast, sinks, out, fixed, fixed_bytes);
   }
 }
 
@@ -1034,17 +805,6 @@ SplitDecArgs split_args(const KvSplit *s, const float *q) {
   a.q_out = nullptr;
   a.tail_w = nullptr;
   return a;
-}
-
-// Notes the stream of a call on the cache.
-void touch(const KvSplit *cs, const Ctx *ctx) {
-  KvSplit *s = const_cast<KvSplit *>(cs);
-  if (s->spread.load(std::memory_order_relaxed)) return;
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) (void)hipGetLastError();
-  hipStream_t first = kNoStream;
-  const bool same = s->stream.compare_exchange_strong(first, ctx->stream) || first == ctx->stream;
-  if (!same || capture != hipStreamCaptureStatusNone) s->spread.store(true);
 }
 
 // Seals the prefix into the handle's buffers, which grow when they are too
@@ -1095,7 +855,6 @@ int seal_into(Ctx *ctx, KvSplit *s, const float *prefix_k, const float *v, size_
   if (flags[1]) return set_error(FOCR_E_VALUE, "nonfinite or incomplete KV group");
   if (flags[2])
     return set_error(FOCR_E_VALUE, s->bits == 8 ? "Q8 KV conversion overflow" : "Q16 KV conversion overflow");
-  touch(s, ctx);
   return FOCR_OK;
 }
 
@@ -1143,11 +902,8 @@ int focr_kv_reseal(focr_ctx *handle, focr_kv_split *kv, const float *prefix_k, c
   FOCR_REQUIRE(prefix_len * s->n_kv * kRecord / 256 < (size_t(1) << 31), FOCR_E_SHAPE,
                "split prefix too long for one seal launch");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  // Work on the old records that this stream does not order before the seal.
-  const hipStream_t used = s->stream.load();
-  if (s->spread.load() || (used != kNoStream && used != ctx->stream)) FOCR_HIP_CHECK(hipDeviceSynchronize());
-  s->stream.store(kNoStream);
-  s->spread.store(false);
+  // Calls on any stream, or captured graphs, may still read the old records.
+  if (s->used.exchange(false)) FOCR_HIP_CHECK(hipDeviceSynchronize());
   const int rc = seal_into(ctx, s, prefix_k, v, prefix_len, capacity);
   if (rc != FOCR_OK) s->prefix_len = s->capacity = s->tail_len = 0;  // nothing to attend over or append to
   return rc;
@@ -1160,7 +916,7 @@ int focr_kv_append(focr_ctx *handle, focr_kv_split *kv, const float *k, const fl
   if (rows == 0) return FOCR_OK;
   FOCR_REQUIRE(s->prefix_len + s->tail_len + rows <= s->capacity, FOCR_E_SHAPE, "split tail capacity");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  touch(s, ctx);
+  s->used.store(true, std::memory_order_relaxed);
   AppendArgs a{k, v, s->tail, s->n_kv, static_cast<int>(s->capacity - s->prefix_len), static_cast<int>(s->tail_len),
                static_cast<int>(rows), static_cast<int>(s->tail_bytes)};
   const int threads = static_cast<int>(rows) * s->n_kv * kTail;
@@ -1182,7 +938,7 @@ int focr_kv_qkv_rows(focr_ctx *handle, focr_kv_split *kv, const float *qkv, size
   FOCR_REQUIRE(rows <= 8, FOCR_E_SHAPE, "decode takes 1..=8 rows");
   FOCR_REQUIRE(s->prefix_len + s->tail_len + rows <= s->capacity, FOCR_E_SHAPE, "split tail capacity");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  touch(s, ctx);
+  s->used.store(true, std::memory_order_relaxed);
   RowAppendArgs a{qkv, rope, q, s->tail, s->n_heads, s->n_kv, static_cast<int>(s->capacity - s->prefix_len),
                   static_cast<int>(s->tail_len), static_cast<int>(s->tail_bytes)};
   if (s->bits == 8)
@@ -1204,7 +960,7 @@ int focr_kv_decode_row(focr_ctx *handle, focr_kv_split *kv, const float *qkv, co
   FOCR_REQUIRE(s->prefix_len + s->tail_len + 1 <= s->capacity, FOCR_E_SHAPE, "split tail capacity");
   FOCR_REQUIRE(s->n_heads == 2 * s->n_kv, FOCR_E_SHAPE, "split decode: two query heads per KV head");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  touch(s, ctx);
+  s->used.store(true, std::memory_order_relaxed);
   SplitDecArgs a = split_args(s, nullptr);
   a.last += 1;  // the new row is position prefix_len + tail_len
   a.qkv = qkv;
@@ -1225,7 +981,7 @@ int focr_kv_attention_decode(focr_ctx *handle, const focr_kv_split *kv, const fl
   FOCR_REQUIRE(rows >= 1 && rows <= 8 && rows <= (s->tail_len > 0 ? s->tail_len : 1), FOCR_E_SHAPE,
                "split decode: 1 to 8 rows, at most the appended positions");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  touch(s, ctx);
+  s->used.store(true, std::memory_order_relaxed);
   const SplitDecArgs a = split_args(s, q);
   const int r = static_cast<int>(rows);
   return s->bits == 8 ? launch_split_rows<int8_t>(ctx, a, r, s->fast_exp, sinks, out, nullptr, 0)
@@ -1240,7 +996,7 @@ int focr_kv_attention_decode_noalloc(focr_ctx *handle, const focr_kv_split *kv, 
   FOCR_REQUIRE(rows >= 1 && rows <= 8 && rows <= (s->tail_len > 0 ? s->tail_len : 1), FOCR_E_SHAPE,
                "split decode: 1 to 8 rows, at most the appended positions");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  touch(s, ctx);
+  s->used.store(true, std::memory_order_relaxed);
   float *fixed = noalloc_scratch(ctx->device);
   FOCR_REQUIRE(fixed, FOCR_E_HIP, "the no-alloc scratch of this device was not resolved (focr_ctx_create does it)");
   const SplitDecArgs a = split_args(s, q);
@@ -1255,7 +1011,7 @@ int focr_kv_dequantize(focr_ctx *handle, const focr_kv_split *kv, float *prefix_
   FOCR_REQUIRE(ctx && s && prefix_k && values && (generated_k || s->tail_len == 0), FOCR_E_ARG,
                "focr_kv_dequantize: null argument");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  touch(s, ctx);
+  s->used.store(true, std::memory_order_relaxed);
   DequantArgs a{s->records, s->tail, prefix_k, values, generated_k, static_cast<int>(s->prefix_len),
                 static_cast<int>(s->tail_len), static_cast<int>(s->capacity - s->prefix_len), s->n_heads, s->n_kv,
                 static_cast<int>(s->record_bytes), static_cast<int>(s->tail_bytes)};

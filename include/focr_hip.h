@@ -321,8 +321,8 @@ int focr_kv_seal(focr_ctx *ctx, int bits, const float *prefix_k_dev, const float
                  size_t head_dim, focr_kv_split **out);
 /* focr_kv_seal into an existing handle (its bits and heads): its old prefix
  * and tail are dropped, its buffers are kept where they are large enough, so
- * a session's next page allocates nothing. Waits for work queued on the old
- * records from other streams or captured graphs. After an error the handle
+ * a session's next page allocates nothing. Waits for the device if any call
+ * has used the old records. After an error the handle
  * holds no prefix and may only be resealed or freed. No reference counterpart
  * (device state). */
 int focr_kv_reseal(focr_ctx *ctx, focr_kv_split *kv, const float *prefix_k_dev, const float *v_dev,
