@@ -978,6 +978,7 @@ int focr_kv_attention_decode(focr_ctx *handle, const focr_kv_split *kv, const fl
   Ctx *ctx = reinterpret_cast<Ctx *>(handle);
   const KvSplit *s = reinterpret_cast<const KvSplit *>(kv);
   FOCR_REQUIRE(ctx && s && q && sinks && out, FOCR_E_ARG, "focr_kv_attention_decode: null argument");
+  FOCR_REQUIRE(s->prefix_len > 0, FOCR_E_SHAPE, "split decode: no sealed prefix (its reseal was refused)");
   FOCR_REQUIRE(rows >= 1 && rows <= 8 && rows <= (s->tail_len > 0 ? s->tail_len : 1), FOCR_E_SHAPE,
                "split decode: 1 to 8 rows, at most the appended positions");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
@@ -993,6 +994,7 @@ int focr_kv_attention_decode_noalloc(focr_ctx *handle, const focr_kv_split *kv, 
   Ctx *ctx = reinterpret_cast<Ctx *>(handle);
   const KvSplit *s = reinterpret_cast<const KvSplit *>(kv);
   FOCR_REQUIRE(ctx && s && q && sinks && out, FOCR_E_ARG, "focr_kv_attention_decode_noalloc: null argument");
+  FOCR_REQUIRE(s->prefix_len > 0, FOCR_E_SHAPE, "split decode: no sealed prefix (its reseal was refused)");
   FOCR_REQUIRE(rows >= 1 && rows <= 8 && rows <= (s->tail_len > 0 ? s->tail_len : 1), FOCR_E_SHAPE,
                "split decode: 1 to 8 rows, at most the appended positions");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
@@ -1010,6 +1012,7 @@ int focr_kv_dequantize(focr_ctx *handle, const focr_kv_split *kv, float *prefix_
   const KvSplit *s = reinterpret_cast<const KvSplit *>(kv);
   FOCR_REQUIRE(ctx && s && prefix_k && values && (generated_k || s->tail_len == 0), FOCR_E_ARG,
                "focr_kv_dequantize: null argument");
+  FOCR_REQUIRE(s->prefix_len > 0, FOCR_E_SHAPE, "focr_kv_dequantize: no sealed prefix (its reseal was refused)");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
   s->used.store(true, std::memory_order_relaxed);
   DequantArgs a{s->records, s->tail, prefix_k, values, generated_k, static_cast<int>(s->prefix_len),

@@ -144,6 +144,19 @@ def test_reseal_is_bitwise_a_fresh_seal(fh, bits):
     with pytest.raises(fh.FocrError, match="nonfinite"):
         kv.reseal(kd, to_dev(nan), P, cap)
     assert kv.handle is None
+    # A refused handle attends over nothing: the C entries refuse it, and it
+    # can be resealed.
+    kv = fh.KvSplit.seal(bits, kd, vd, P, cap, N_HEADS, N_KV)
+    lib, bad = fh.lib(), to_dev(nan)
+    assert lib.focr_kv_reseal(ctx.handle, kv.handle, kd.data_ptr(), bad.data_ptr(), P, cap) != 0
+    out = torch.empty_like(q[:1])
+    with pytest.raises(fh.FocrError, match="no sealed prefix"):
+        kv.attention_decode(q[:1], 1, sinks)
+    assert lib.focr_kv_attention_decode_noalloc(ctx.handle, kv.handle, q.data_ptr(), 1, sinks.data_ptr(), out.data_ptr()) != 0
+    assert lib.focr_kv_reseal(ctx.handle, kv.handle, kd.data_ptr(), vd.data_ptr(), P, cap) == 0
+    for got, want in zip(kv.dequantize()[:2], fh.KvSplit.seal(bits, kd, vd, P, cap, N_HEADS, N_KV).dequantize()[:2]):
+        assert_bitwise(host(got), host(want))
+    kv.free()
 
 
 @pytest.mark.parametrize("fast", [False, True])
