@@ -37,6 +37,7 @@
 #include <atomic>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "decode_common.hpp"
@@ -115,43 +116,51 @@ __device__ __forceinline__ uint16_t bf16_up(float scale) {
 }
 
 // round_clamped(value / step): clamp to +-limit in f64, round to nearest
-// even; NaN gives 0 (Rust's saturating cast); a zero step gives 0.
-__device__ __forceinline__ int code_of(float value, float step, double limit) {
+// even; NaN gives 0 (Rust's saturating cast); a zero step gives 0. In FP32:
+// value * rcp(step) lies within 0.02 of the quotient (|quotient| < 2^15), so
+// its nearest integer n is the code or next to it, and the remainder
+// value - n * step, which one FMA forms exactly (a BF16 step has 8 bits, so
+// n * step has 23, and with |remainder| <= |value| it is a whole number of
+// the value's units; n = 0 leaves the value), decides: past half a step, or a
+// tie at an odd n, moves n towards it. The same as the f64 quotient rounds
+// to: a quotient off a tie is off by 2^-31 of itself or more. Steps below
+// 2^-100, where reciprocals overflow and units vanish, keep the f64 quotient.
+__device__ __forceinline__ int code_of(float value, float step, float limit) {
   if (step == 0.0f) return 0;
+  if (!(step < 7.888609e-31f)) {
+    float n = __builtin_rintf(value * __builtin_amdgcn_rcpf(step));
+    const float rest = fmaf_(-n, step, value), twice = 2.0f * fabsf(rest);
+    if (twice > step || (twice == step && (static_cast<int>(n) & 1))) n += __builtin_copysignf(1.0f, rest);
+    n = n < -limit ? -limit : (n > limit ? limit : n);
+    return n == n ? static_cast<int>(n) : 0;
+  }
   double x = static_cast<double>(value) / static_cast<double>(step);
   if (x != x) return 0;
-  x = x < -limit ? -limit : (x > limit ? limit : x);
+  const double top = limit;
+  x = x < -top ? -top : (x > top ? top : x);
   return static_cast<int>(rint(x));
 }
 
+// The step of a block with largest magnitude mx (q8_scale / q16_scale): mx /
+// limit in f64 rounded to f32 (the FP32 quotient: 53 bits are more than twice
+// 24, so rounding twice is rounding once), at least the smallest subnormal, 0
+// for an all-zero block.
+__device__ __forceinline__ float block_step(float mx, float limit) {
+  if (mx == 0.0f) return 0.0f;
+  const float step = mx / limit;
+  return step > 1.40129846e-45f ? step : 1.40129846e-45f;
+}
+
 // Codes one 32-element block held by the 32 lanes of a half-wave (lane & 31
-// = element; every lane of the wave takes part in the exchanges). The step
-// (q8_scale / q16_scale) is absmax / limit in f64 rounded to f32, at least
-// the smallest subnormal, 0 for an all-zero block, stored as the smallest
-// BF16 at or above it; `nan_step` stores the NaN pattern instead. The max is
-// exact, so the exchange order does not matter. Returns the code; `step`
-// receives the stored BF16. DPP: the exchanges by v_permlane16_swap (the
-// half's two rows) and DPP within the rows instead of five LDS permutes.
-template <bool DPP = false>
-__device__ __forceinline__ int code_lane(float x, bool nan_step, double limit, uint16_t &stored) {
+// = element; every lane of the wave takes part in the exchanges). The step is
+// stored as the smallest BF16 at or above it; `nan_step` stores the NaN
+// pattern instead. The max is exact, so the exchange order does not matter.
+// Returns the code; `stored` receives the BF16.
+__device__ __forceinline__ int code_lane(float x, bool nan_step, float limit, uint16_t &stored) {
   float mx = __builtin_fmaxf(0.0f, fabsf(x));  // a NaN element counts as 0
-  if constexpr (DPP) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-    mx = __builtin_fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));  // lanes i and i ^ 16
-    mx = __builtin_fmaxf(mx, dpp<0xB1>(mx));   // quad_perm [1,0,3,2]
-    mx = __builtin_fmaxf(mx, dpp<0x4E>(mx));   // quad_perm [2,3,0,1]
-    mx = __builtin_fmaxf(mx, dpp<0x141>(mx));  // row_half_mirror
-    mx = __builtin_fmaxf(mx, dpp<0x140>(mx));  // row_mirror
-  } else {
 #pragma unroll
-    for (int mask = 1; mask < 32; mask *= 2) mx = __builtin_fmaxf(mx, xor_lane(mx, mask));
-  }
-  float step = 0.0f;
-  if (mx != 0.0f) {
-    step = static_cast<float>(static_cast<double>(mx) / limit);
-    step = step > 1.40129846e-45f ? step : 1.40129846e-45f;
-  }
-  stored = bf16_up(nan_step ? __builtin_nanf("") : step);
+  for (int mask = 1; mask < 32; mask *= 2) mx = __builtin_fmaxf(mx, xor_lane(mx, mask));
+  stored = bf16_up(nan_step ? __builtin_nanf("") : block_step(mx, limit));
   return code_of(x, bf16_widen(stored), limit);
 }
 
@@ -171,46 +180,81 @@ struct SealArgs {
 };
 
 // Records per seal_kernel lane.
-constexpr int kSealPer = 8;
+constexpr int kSealPer = 4;
 
-// Lane = element e of kSealPer records, `pass` records apart (group-major
-// records of 160 = 5 blocks of 32, so every block is one aligned half-wave):
-// gathers the elements (every load issued before any element is coded, so
-// a wave has kSealPer loads in flight instead of one), checks the pair
-// sharing (block 0) and finiteness, codes them.
-template <typename C>
-__global__ __launch_bounds__(256) void seal_kernel(SealArgs a, long pass) {
-  const long idx = static_cast<long>(blockIdx.x) * 256 + threadIdx.x;
-  const long nrec = static_cast<long>(a.n_kv) * a.prefix_len;
-  const long rec0 = idx / kRecord;
-  const int e = static_cast<int>(idx % kRecord);
-  float x[kSealPer], pair[kSealPer];
+// Lane = four neighbouring elements of kSealPer records of group blockIdx.y,
+// `pass` positions apart; a block of 32 is eight lanes (records of 160 = 5
+// blocks). Gathers the elements (16-byte loads where the caller's buffers
+// allow, VEC; every load issued before any element is coded), checks the pair
+// sharing (block 0) and finiteness, codes them, one store per lane.
+// Bound: VALU issue before HBM. The f64 quotients of step and code, a 64-bit
+// division per record for its position, and a lane per element that stored
+// one code had taken most of it: 6,544
+// positions of 8 groups, Q8, 33.2 -> 17.2 us (2.9 TB/s), 1,501 of Q16 12.6 ->
+// 7.7 us.
+template <typename C, bool VEC>
+__global__ __launch_bounds__(256) void seal_kernel(SealArgs a, int pass) {
+  constexpr int kBlocks = kRecord / 32;
+  const uint32_t run = blockIdx.x * 32u + (threadIdx.x >> 3);  // block of 32 elements
+  const int rec0 = static_cast<int>(run / kBlocks), g = blockIdx.y;
+  const int e = static_cast<int>(run % kBlocks) * 32 + 4 * (threadIdx.x & 7);
+  const size_t group = static_cast<size_t>(g) * a.prefix_len;
+  float x[kSealPer][4], pair[kSealPer][4];
   bool valid[kSealPer];
+  auto load = [](float *dst, const float *src) __attribute__((always_inline)) {
+    if constexpr (VEC) {
+      const float4 t = ld4(src);
+      dst[0] = t.x;
+      dst[1] = t.y;
+      dst[2] = t.z;
+      dst[3] = t.w;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++) dst[i] = src[i];
+    }
+  };
 #pragma unroll
   for (int j = 0; j < kSealPer; j++) {
-    const long record = rec0 + j * pass;
-    valid[j] = rec0 < pass && record < nrec;
-    const long r = valid[j] ? record : 0;
-    const int g = static_cast<int>(r / a.prefix_len), t = static_cast<int>(r % a.prefix_len);
+    valid[j] = rec0 < pass && rec0 + static_cast<long>(j) * pass < a.prefix_len;
+    const int t = valid[j] ? rec0 + j * pass : 0;
     const float *ka = a.k + (static_cast<size_t>(t) * a.n_heads + 2 * g) * 64;
     const float *src =
         e < 64 ? ka + e : e < 96 ? ka + 32 + e : a.v + (static_cast<size_t>(t) * a.n_kv + g) * 64 + e - 96;
-    x[j] = valid[j] ? *src : 0.0f;
-    pair[j] = valid[j] && e < 32 ? ka[64 + e] : 0.0f;
+    load(x[j], src);
+    if (e < 32) load(pair[j], ka + 64 + e);
   }
   uint32_t err = 0;
-  const double limit = sizeof(C) == 1 ? 127.0 : 32767.0;
+  const float limit = sizeof(C) == 1 ? 127.0f : 32767.0f;
 #pragma unroll
   for (int j = 0; j < kSealPer; j++) {
-    if (valid[j] && !__builtin_isfinite(x[j])) err |= kErrNonFinite;
-    if (valid[j] && e < 32 && __float_as_uint(x[j]) != __float_as_uint(pair[j])) err |= kErrPair;
-    uint16_t stored;
-    const int code = code_lane<true>(x[j], false, limit, stored);
+    float mx = 0.0f;  // a NaN element counts as 0
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      mx = __builtin_fmaxf(mx, fabsf(x[j][i]));
+      if (valid[j] && !__builtin_isfinite(x[j][i])) err |= kErrNonFinite;
+      if (valid[j] && e < 32 && __float_as_uint(x[j][i]) != __float_as_uint(pair[j][i])) err |= kErrPair;
+    }
+    mx = __builtin_fmaxf(mx, dpp<0xB1>(mx));   // quad_perm [1,0,3,2]
+    mx = __builtin_fmaxf(mx, dpp<0x4E>(mx));   // quad_perm [2,3,0,1]
+    mx = __builtin_fmaxf(mx, dpp<0x141>(mx));  // row_half_mirror
+    const uint16_t stored = bf16_up(block_step(mx, limit));
+    const float step = bf16_widen(stored);
+    int code[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      code[i] = code_of(x[j][i], step, limit);
+      if (valid[j] && !__builtin_isfinite(static_cast<float>(code[i]) * step)) err |= kErrOverflow;
+    }
     if (valid[j]) {
-      unsigned char *rec = a.records + static_cast<size_t>(rec0 + j * pass) * a.record_bytes;
-      reinterpret_cast<C *>(rec)[e] = static_cast<C>(code);
+      unsigned char *rec = a.records + (group + rec0 + j * pass) * a.record_bytes;
+      if constexpr (sizeof(C) == 1)
+        *reinterpret_cast<uint32_t *>(rec + e) =
+            (code[0] & 0xff) | (code[1] & 0xff) << 8 | (code[2] & 0xff) << 16 | static_cast<uint32_t>(code[3]) << 24;
+      else
+        *reinterpret_cast<uint2 *>(rec + 2 * e) =
+            make_uint2((code[0] & 0xffff) | static_cast<uint32_t>(code[1]) << 16,
+                       (code[2] & 0xffff) | static_cast<uint32_t>(code[3]) << 16);
       if ((e & 31) == 0) reinterpret_cast<uint16_t *>(rec + kRecord * sizeof(C))[e >> 5] = stored;
-      if (!__builtin_isfinite(static_cast<float>(code) * bf16_widen(stored))) err |= kErrOverflow;
     }
   }
   if (err & kErrPair) a.error[0] = 1;
@@ -235,7 +279,7 @@ __global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
   const float x = valid ? *src : 0.0f;
   const bool nonfinite = half_any(!__builtin_isfinite(x));
   uint16_t stored;
-  const int code = code_lane(x, nonfinite, sizeof(C) == 1 ? 127.0 : 32767.0, stored);
+  const int code = code_lane(x, nonfinite, sizeof(C) == 1 ? 127.0f : 32767.0f, stored);
   if (valid) {
     unsigned char *rec = a.tail + (static_cast<size_t>(g) * a.tail_capacity + a.first + r) * a.tail_bytes;
     reinterpret_cast<C *>(rec)[e] = static_cast<C>(code);
@@ -268,7 +312,7 @@ __global__ __launch_bounds__(1024) void row_append_kernel(RowAppendArgs a) {
   const int qdim = a.n_heads * 64, kdim = a.n_kv * 64, repeat = a.n_heads / a.n_kv;
   const float *src = a.qkv + static_cast<size_t>(row) * (qdim + 2 * kdim);
   const float2 *rope = reinterpret_cast<const float2 *>(a.rope) + static_cast<size_t>(row) * a.n_heads * 32;
-  const double limit = sizeof(C) == 1 ? 127.0 : 32767.0;
+  const float limit = sizeof(C) == 1 ? 127.0f : 32767.0f;
   const int jobs = a.n_heads + 2 * a.n_kv;
   // Job j: query head j, key head j - n_heads, or the values of group
   // j - n_heads - n_kv.
@@ -512,7 +556,7 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
       const float x = key ? a.qkv[qdim + g * 64 + lane] : a.qkv[qdim + kdim + g * 64 + lane];
       const float y = key ? norm_rope(x, rope[g * repeat * 32 + lane / 2], lane) : x;
       uint16_t stored;
-      const int code = code_lane(y, half_any(!__builtin_isfinite(y)), sizeof(C) == 1 ? 127.0 : 32767.0, stored);
+      const int code = code_lane(y, half_any(!__builtin_isfinite(y)), sizeof(C) == 1 ? 127.0f : 32767.0f, stored);
       unsigned char *rec = a.tail_w + static_cast<size_t>(g) * a.tail_capacity * a.tail_bytes;
       const int el = (key ? 0 : 64) + lane;
       reinterpret_cast<C *>(rec)[el] = static_cast<C>(code);
@@ -839,14 +883,22 @@ int seal_into(Ctx *ctx, KvSplit *s, const float *prefix_k, const float *v, size_
   flags[0] = flags[1] = flags[2] = 0;
   SealArgs a{prefix_k, v, s->records, ctx->flags, static_cast<int>(prefix_len), s->n_heads, s->n_kv,
              static_cast<int>(s->record_bytes)};
-  const long nrec = static_cast<long>(s->n_kv) * prefix_len;
-  const long pass = (nrec + kSealPer - 1) / kSealPer;
-  const dim3 grid(static_cast<unsigned>((pass * kRecord + 255) / 256));
-  static_assert(kRecord % 32 == 0 && kTail % 64 == 0, "blocks are whole half-waves");
-  if (s->bits == 8)
-    hipLaunchKernelGGL(seal_kernel<int8_t>, grid, dim3(256), 0, ctx->stream, a, pass);
+  const int pass = static_cast<int>((prefix_len + kSealPer - 1) / kSealPer);
+  const dim3 grid(static_cast<unsigned>((static_cast<size_t>(pass) * (kRecord / 4) + 255) / 256),
+                  static_cast<unsigned>(s->n_kv));
+  static_assert(kRecord % 32 == 0 && kTail % 64 == 0, "blocks are whole groups of eight lanes and half-waves");
+  const bool vec = ((reinterpret_cast<uintptr_t>(prefix_k) | reinterpret_cast<uintptr_t>(v)) & 15) == 0;
+  auto launch = [&](auto code, auto wide) {
+    hipLaunchKernelGGL((seal_kernel<decltype(code), decltype(wide)::value>), grid, dim3(256), 0, ctx->stream, a, pass);
+  };
+  if (s->bits == 8 && vec)
+    launch(int8_t(), std::true_type());
+  else if (s->bits == 8)
+    launch(int8_t(), std::false_type());
+  else if (vec)
+    launch(int16_t(), std::true_type());
   else
-    hipLaunchKernelGGL(seal_kernel<int16_t>, grid, dim3(256), 0, ctx->stream, a, pass);
+    launch(int16_t(), std::false_type());
   e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) return set_error(FOCR_E_HIP, std::string("focr_kv_seal: ") + hipGetErrorString(e));

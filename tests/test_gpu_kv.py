@@ -89,6 +89,33 @@ def test_tiny_subnormal_and_zero_blocks_are_bitwise_the_oracle(fh, bits):
     kv.free()
 
 
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("bits", [8, 16])
+def test_codes_at_and_beside_ties_are_bitwise_the_oracle(fh, bits, shift):
+    # Blocks whose step is a BF16 value exactly (their largest value is limit
+    # steps) from 2^-120 to 2^100 on both sides of the 2^-100 line between the
+    # FP32 and the f64 quotient: every value is (n + 1/2) steps or a neighbour
+    # of that, n over the whole range of codes. Records and tail; buffers 16-byte
+    # aligned and one float off that.
+    limit = 127 if bits == 8 else 32767
+    rng = np.random.Generator(np.random.PCG64(17))
+    P, rows, blocks = 517, 8, N_KV * 2
+    exps = rng.integers(-127, 93, size=(P + rows, blocks, 1))
+    step = np.ldexp(rng.integers(128, 256, size=exps.shape).astype(F32), exps).astype(F32)
+    n = rng.integers(-limit, limit, size=(P + rows, blocks, 32))
+    v = ((n + 0.5) * step.astype(np.float64)).astype(F32)
+    v = (v.view(np.int32) + rng.integers(-1, 2, size=v.shape).astype(np.int32)).view(F32)
+    v[:, :, 5] = (limit * step[:, :, 0].astype(np.float64)).astype(F32)
+    v = v.reshape(P + rows, N_KV, 64)
+    k, _ = pair_cache(P, N_KV, 18, 2.0)
+    kd, vd = (to_dev(np.concatenate([np.zeros(shift, F32), x.reshape(-1)]))[shift:] for x in (k, v[:P]))
+    kv = fh.KvSplit.seal(bits, kd, vd, P, P + rows, N_HEADS, N_KV)
+    kv.append(to_dev(v[P:]), to_dev(v[P:]), rows)
+    for got, want in zip(kv.dequantize(), oracle_cache(bits, k, v[:P], P, v[P:], v[P:], P + rows)):
+        assert_bitwise(host(got), want)
+    kv.free()
+
+
 def test_refusals(fh):
     P = 6
     k, v = pair_cache(P, N_KV, 21)
