@@ -1028,22 +1028,27 @@ union PairFrag {
   pair_half8 v;
 };
 
-// 128 x 128 outputs per workgroup, 4 waves in 2 x 2, each 64 x 64 in 32 x 32
-// blocks. Stages of 16 k: per operand two planes x 128 rows x 32 bytes
+// BM x 128 outputs per workgroup, 4 waves in 2 x 2, each BM / 2 x 64 in 32 x 32
+// blocks. Stages of 16 k: per operand two planes x its rows x 32 bytes
 // (each plane's rows of a stage contiguous in memory), copied HBM -> LDS by
-// the LDS-DMA path (16 bytes per lane, two copies of 1 KB per wave and
-// operand) into a ring of three stages, two stages ahead. A row's
+// the LDS-DMA path (16 bytes per lane, copies of 1 KB) into a ring of three
+// stages, two stages ahead. A row's
 // two 16-byte chunks (k 0..7, 8..15) are stored swapped when (row / 8) is
 // odd: the 16 lanes a ds_read_b128 serves (rows r..r+15, one chunk) then hit
 // 16 distinct bank groups. Step st reads stage st's fragments while the
 // products of stage st - 1 run. Rows and columns are padded to 128 with zeros
 // in the planes; outputs past m or n are not written.
+// Bound: the LDS and the barrier per stage beside the matrix cores. A 128-row
+// tile's stage reads 64 KB of fragments per compute unit and writes 32 KB for
+// 768 matrix-core cycles per SIMD, as many as the LDS takes; a 256-row tile's
+// takes 0.75 of that per product and has half the barriers. It holds 256
+// VGPRs (held to two waves per SIMD, a few values spilled).
 template <int EPI, int BM>
-__global__ __launch_bounds__(256) void split_kernel(GemmArgs a, const uint16_t *__restrict__ ap,
+__global__ __launch_bounds__(256, BM == 256 ? 2 : 1) void split_kernel(GemmArgs a, const uint16_t *__restrict__ ap,
                                                     const uint16_t *__restrict__ bp, const int *__restrict__ aexp,
                                                     const int *__restrict__ bexp, size_t a_plane, size_t b_plane,
                                                     int kp, int row_tiles, int col_tiles) {
-  // BM x 128 outputs (BM = 128 or 64). An A plane of a stage holds 2 BM
+  // BM x 128 outputs (BM = 256, 128 or 64). An A plane of a stage holds 2 BM
   // slots of 16 bytes (AS), a B plane 256. The ring's three slots, each
   // [A plane * AS + slot u | B plane * 256 + slot u], are separate arrays and
   // every step names its slots statically: the compiler then sees that a
@@ -1052,8 +1057,9 @@ __global__ __launch_bounds__(256) void split_kernel(GemmArgs a, const uint16_t *
   constexpr int IB = BM / 64;               // 32-row blocks per wave
   constexpr int RS = 2 * AS + 2 * 256;  // slots of one ring entry
   __shared__ uint4 ring0[RS], ring1[RS], ring2[RS];
-  __shared__ int tile_exp[2][kSplitBN];
-  __shared__ bool tile_bad[2][kSplitBN];
+  constexpr int TE = BM > kSplitBN ? BM : kSplitBN;
+  __shared__ int tile_exp[2][TE];
+  __shared__ bool tile_bad[2][TE];
   __shared__ int tile_any;  // a flagged row or column in the tile
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -1065,19 +1071,20 @@ __global__ __launch_bounds__(256) void split_kernel(GemmArgs a, const uint16_t *
   // Copy t of operand o fills slots q = 64 (wave + 4 t) + lane: plane q / S,
   // slot u = q % S = row u / 2, chunk (u % 2) ^ ((row / 8) % 2) (S = AS for
   // A, 256 for B).
-  const char *src[2][2];
+  const char *asrc[AC], *bsrc[2];
+#pragma unroll
+  for (int t = 0; t < AC; t++) {
+    const int q = 64 * (wave + 4 * t) + lane;
+    const int pa = q / AS, ua = q % AS, ra = ua >> 1;
+    const int ca = (ua & 1) ^ ((ra >> 3) & 1);
+    asrc[t] = reinterpret_cast<const char *>(ap + pa * a_plane + static_cast<size_t>(m0 + ra) * kSplitBK + 8 * ca);
+  }
 #pragma unroll
   for (int t = 0; t < 2; t++) {
     const int q = 64 * (wave + 4 * t) + lane;
-    {
-      const int pa = q / AS, ua = q % AS, ra = ua >> 1;
-      const int ca = (ua & 1) ^ ((ra >> 3) & 1);
-      src[0][t] = reinterpret_cast<const char *>(ap + (pa < 2 ? pa : 1) * a_plane +
-                                                 static_cast<size_t>(m0 + ra) * kSplitBK + 8 * ca);
-    }
     const int pb = q >> 8, ub = q & 255, rb = ub >> 1;
     const int cb = (ub & 1) ^ ((rb >> 3) & 1);
-    src[1][t] = reinterpret_cast<const char *>(bp + pb * b_plane + static_cast<size_t>(n0 + rb) * kSplitBK + 8 * cb);
+    bsrc[t] = reinterpret_cast<const char *>(bp + pb * b_plane + static_cast<size_t>(n0 + rb) * kSplitBK + 8 * cb);
   }
   const int stages = kp / kSplitBK;  // even
   // Stage-major planes: stage s of a plane starts rows_pad * 32 bytes after s - 1.
@@ -1085,11 +1092,11 @@ __global__ __launch_bounds__(256) void split_kernel(GemmArgs a, const uint16_t *
   auto issue = [&](uint4 *slot, int stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < AC; t++)
-      __builtin_amdgcn_global_load_lds((global_void *)(src[0][t] + stage * a_step),
+      __builtin_amdgcn_global_load_lds((global_void *)(asrc[t] + stage * a_step),
                                        (lds_void *)(&slot[64 * (wave + 4 * t)]), 16, 0, 0);
 #pragma unroll
     for (int t = 0; t < 2; t++)
-      __builtin_amdgcn_global_load_lds((global_void *)(src[1][t] + stage * b_step),
+      __builtin_amdgcn_global_load_lds((global_void *)(bsrc[t] + stage * b_step),
                                        (lds_void *)(&slot[2 * AS + 64 * (wave + 4 * t)]), 16, 0, 0);
   };
   // Fragments of a stage: A blocks i and B blocks j, planes hi, lo.
@@ -1164,12 +1171,12 @@ __global__ __launch_bounds__(256) void split_kernel(GemmArgs a, const uint16_t *
   products(fa1, fb1);
   // The tile's row and column exponents (the planes are padded to whole
   // 128-row tiles, and so are the exponent arrays) and non-finite flags.
-  if (tid < BM || tid >= 128) {
-    const int o = tid < BM ? 0 : 1, t = tid & 127;
-    const int e = o == 0 ? aexp[m0 + t] : bexp[n0 + t];
+  for (int t = tid; t < BM + kSplitBN; t += 256) {
+    const int o = t < BM ? 0 : 1, u = o == 0 ? t : t - BM;
+    const int e = o == 0 ? aexp[m0 + u] : bexp[n0 + u];
     const bool bad = e >= kPairNonfinite / 2;
-    tile_exp[o][t] = bad ? e - kPairNonfinite : e;
-    tile_bad[o][t] = bad;
+    tile_exp[o][u] = bad ? e - kPairNonfinite : e;
+    tile_bad[o][u] = bad;
     if (bad) tile_any = 1;
   }
   // The repeated copies must land before the workgroup's LDS is released.
@@ -1361,30 +1368,19 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
   GemmArgs a = make_args(lin, x, rows, row_scale, out);
   const int ctiles = static_cast<int>(n_pad / kSplitBN), rt128 = static_cast<int>(m_pad / kSplitBM);
   const int k32 = static_cast<int>(kp);
-  auto launch = [&](int bm, int row0, int rtiles) {
+  auto launch = [&](auto bm, int row0, int rtiles) {
+    constexpr int BM = decltype(bm)::value;
     a.row0 = row0;
     const dim3 grid(static_cast<unsigned>(rtiles * ctiles));
-    if (bm == 128) {
-      if (epilogue == FOCR_EPI_GLU)
-        hipLaunchKernelGGL((split_kernel<FOCR_EPI_GLU, 128>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp, bexp,
-                           a_plane, b_plane, k32, rtiles, ctiles);
-      else if (epilogue == FOCR_EPI_ADD)
-        hipLaunchKernelGGL((split_kernel<FOCR_EPI_ADD, 128>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp, bexp,
-                           a_plane, b_plane, k32, rtiles, ctiles);
-      else
-        hipLaunchKernelGGL((split_kernel<FOCR_EPI_STORE, 128>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp,
-                           bexp, a_plane, b_plane, k32, rtiles, ctiles);
-    } else {
-      if (epilogue == FOCR_EPI_GLU)
-        hipLaunchKernelGGL((split_kernel<FOCR_EPI_GLU, 64>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp, bexp,
-                           a_plane, b_plane, k32, rtiles, ctiles);
-      else if (epilogue == FOCR_EPI_ADD)
-        hipLaunchKernelGGL((split_kernel<FOCR_EPI_ADD, 64>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp, bexp,
-                           a_plane, b_plane, k32, rtiles, ctiles);
-      else
-        hipLaunchKernelGGL((split_kernel<FOCR_EPI_STORE, 64>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp,
-                           bexp, a_plane, b_plane, k32, rtiles, ctiles);
-    }
+    if (epilogue == FOCR_EPI_GLU)
+      hipLaunchKernelGGL((split_kernel<FOCR_EPI_GLU, BM>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp, bexp, a_plane,
+                         b_plane, k32, rtiles, ctiles);
+    else if (epilogue == FOCR_EPI_ADD)
+      hipLaunchKernelGGL((split_kernel<FOCR_EPI_ADD, BM>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp, bexp, a_plane,
+                         b_plane, k32, rtiles, ctiles);
+    else
+      hipLaunchKernelGGL((split_kernel<FOCR_EPI_STORE, BM>), grid, dim3(256), 0, ctx->stream, a, ap, bp, aexp, bexp,
+                         a_plane, b_plane, k32, rtiles, ctiles);
   };
   // By 32 x 32 blocks of output (us, this form and its neighbours): 120 (WO,
   // m = 144) 32 x 32 5.7, 32 x 64 7.0; 288 (W13, 48) 32 x 64 6.5, 32 x 32 8.0;
@@ -1421,22 +1417,35 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
     FOCR_HIP_CHECK(hipGetLastError());
     return FOCR_OK;
   }
-  // 128-row tiles fill 512 workgroup slots (two per compute unit, by VGPRs).
-  // Fewer tiles than that run as 64-row tiles (twice as many, half the
-  // work each); when the 128-row tiles' last round would be at most half
-  // full, whole rounds run as 128-row tiles and the rows left as 64-row tiles.
+  // 256- and 128-row tiles fill 512 workgroup slots (two per compute unit, by
+  // VGPRs). 256-row tiles take whole rounds, and all rows where the last round
+  // is at least 0.3 full behind a whole one or 0.8 full as the only one; the
+  // rows left (or all of them) run as 128-row tiles, or as 64-row tiles (twice
+  // as many, half the work each) where those would fill less than 0.8 of their
+  // only round, or at most half of their last one.
+  // us per call, 128- and 64-row tiles alone -> with 256-row tiles: QKV 6,544
+  // (0.81 rounds) 82 -> 79, 16,320 (2.0) 188 -> 175; W13 6,544 (1.83) 169 -> 158,
+  // 12,000 (3.30) 284 -> 261 (267 with only the whole rounds), 16,320 372 -> 349;
+  // 1024 -> 4096 4,000 (1.0) 116 -> 105, 9,000 (2.19) 250 -> 239 (256 with all
+  // rows). Below the lines: W13 4,000 (1.13) 107, 116 with all rows; 2,500 (0.70)
+  // 73 and 76; WO 12,000 (0.55) 92 and 99. 128- against 64-row tiles in one
+  // round of 0.83 (n = 768, 9,000 rows): WO 69 -> 64, W2 153 -> 138.
   constexpr int kSlots = 512;
-  const int tiles = rt128 * ctiles, full = tiles / kSlots;
+  const integral_constant<int, 256> tall;
+  const integral_constant<int, 128> mid;
+  const integral_constant<int, 64> low;
+  const int tall_tiles = rt128 / 2 * ctiles, tall_left = tall_tiles % kSlots;
+  const bool all_tall = 10 * tall_left >= (tall_tiles > kSlots ? 3 : 8) * kSlots;
+  const int tall_rows = all_tall ? rt128 / 2 : (tall_tiles - tall_left) / ctiles;
+  if (tall_rows > 0) launch(tall, 0, tall_rows);
+  const int first = 2 * tall_rows, rest = rt128 - first;  // 128-row tiles
+  const int tiles = rest * ctiles, full = tiles / kSlots;
   const int whole = full * kSlots / ctiles;  // 128-row tiles in whole rounds
-  if (full == 0) {
-    launch(64, 0, static_cast<int>((rows + 63) / 64));
-  } else if (whole < rt128 && (rt128 - whole) * ctiles <= kSlots / 2) {
-    launch(128, 0, whole);
-    FOCR_HIP_CHECK(hipGetLastError());
-    launch(64, whole * kSplitBM, static_cast<int>((rows - static_cast<size_t>(whole) * kSplitBM + 63) / 64));
-  } else {
-    launch(128, 0, rt128);
-  }
+  const bool split_last = whole < rest && (rest - whole) * ctiles <= kSlots / 2;
+  const int mid_rows = full == 0 ? (5 * tiles >= 4 * kSlots ? rest : 0) : split_last ? whole : rest;
+  if (mid_rows > 0) launch(mid, first * kSplitBM, mid_rows);
+  const int low0 = (first + mid_rows) * kSplitBM;
+  if (mid_rows < rest) launch(low, low0, static_cast<int>((rows - static_cast<size_t>(low0) + 63) / 64));
   FOCR_HIP_CHECK(hipGetLastError());
   return FOCR_OK;
 }

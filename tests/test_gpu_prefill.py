@@ -246,6 +246,33 @@ def test_f32_split_tile_heights(fh, m):
     assert_bitwise(add, (base + got).astype(np.float32), "add of store")
 
 
+# 256-row tiles: alone in a round 0.8 full (3,300 rows of 4,096 outputs, ragged
+# rows), one whole round and an odd 128 rows (4,200), whole rounds with the
+# rest as 64-row tiles (5,000) and as 128-row ones (2,900 of 8,192), every row
+# behind a whole round (6,600); and a round of 128-row tiles 0.83 full (9,000
+# of 768). Stage counts around the ring's length.
+@pytest.mark.parametrize("m,k,n", [(3300, 64, 4096), (4200, 32, 4090), (5000, 160, 4096), (2900, 64, 8192), (6600, 96, 4096),
+                                   (9000, 64, 768)])
+def test_f32_split_tall_tiles(fh, m, k, n):
+    oracle.set_threads(oracle_threads())
+    a, w = gen.normal((m, k), 1.0, 47), gen.normal((n, k), 0.02, 48)
+    a[m - 1, 3], w[n - 2, 5] = np.inf, np.nan
+    S = fh.PrefillProjection.F32_SPLIT
+    lin = fh.Linear.from_f32(w)
+    got = run_prefill(fh, lin, a, m, None, fh.Epilogue.STORE, S)
+    want = oracle.panel_gemm_fast(a, m, k, w, n)
+    assert_bitwise(got[m - 1], want[m - 1], "flagged row")
+    assert_bitwise(got[:, n - 2], want[:, n - 2], "flagged column")
+    mag = np.abs(a[:-1].astype(np.float64)) @ np.abs(np.delete(w, n - 2, 0).astype(np.float64)).T
+    diff = np.abs(np.delete(got, n - 2, 1)[:-1].astype(np.float64) - np.delete(want, n - 2, 1)[:-1])
+    assert np.all(diff <= 2 * k * EPS * mag + 1e-30)
+    glu = run_prefill(fh, lin, a, m, None, fh.Epilogue.GLU, S)
+    up = got.reshape(m, n // 2, 2)
+    with np.errstate(invalid="ignore"):  # the flagged row and column pair, not compared
+        plain = (np.maximum(up[..., 0], np.float32(0)) ** 2 * up[..., 1]).astype(np.float32)
+    assert_bitwise(glu[:-1, :-1], plain[:-1, :-1], "glu of store")
+
+
 def test_f32_split_power_of_two_row_scaling_is_exact(fh):
     # Each row of A and of W takes its own power-of-two scale, so scaling row
     # i of A by 2^a_i and row j of W by 2^b_j scales output (i, j) by exactly
