@@ -955,7 +955,15 @@ int focr_kv_reseal(focr_ctx *handle, focr_kv_split *kv, const float *prefix_k, c
                "split prefix too long for one seal launch");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
   // Calls on any stream, or captured graphs, may still read the old records.
-  if (s->used.exchange(false)) FOCR_HIP_CHECK(hipDeviceSynchronize());
+  // A refused wait (a stream being captured) leaves them marked as in use.
+  if (s->used.exchange(false)) {
+    const hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess) {
+      s->used.store(true);
+      (void)hipGetLastError();
+      return set_error(FOCR_E_HIP, std::string("focr_kv_reseal: waiting for the old records' readers: ") + hipGetErrorString(e));
+    }
+  }
   const int rc = seal_into(ctx, s, prefix_k, v, prefix_len, capacity);
   if (rc != FOCR_OK) s->prefix_len = s->capacity = s->tail_len = 0;  // nothing to attend over or append to
   return rc;

@@ -186,6 +186,56 @@ def test_reseal_is_bitwise_a_fresh_seal(fh, bits):
     kv.free()
 
 
+@pytest.mark.parametrize("refused", [False, True])
+@pytest.mark.parametrize("bits", [8, 16])
+def test_reseal_waits_for_readers_on_other_streams(fh, bits, refused):
+    # A decode over the old records is queued behind a clock sleep on another
+    # context's stream when the handle is resealed with other values: it still
+    # reads the old ones. `refused`: a first reseal whose wait for the device is
+    # refused (another stream is being captured) leaves that wait to the second.
+    import ctypes
+
+    import torch
+
+    ctx, lib = fh.default_context(), fh.lib()
+    P, cap, rows = 6544, 6560, 2
+    (k, v), (k2, v2) = (tuple(to_dev(x) for x in pair_cache(P, N_KV, s, 2.0)) for s in (91, 92))
+    tk, tv = to_dev(gen.normal((rows, N_KV, 64), 1.0, 93)), to_dev(gen.normal((rows, N_KV, 64), 1.0, 94))
+    q, sinks = to_dev(gen.normal((rows, N_HEADS, 64), 1.0, 95)), to_dev(gen.uniform(N_HEADS, -2.0, 2.0, 96))
+    kv = fh.KvSplit.seal(bits, k, v, P, cap, N_HEADS, N_KV)
+    kv.append(tk, tv, rows)
+    want = host(kv.attention_decode(q, rows, sinks))
+    other, side, captured = fh.Context(0), torch.cuda.Stream(), torch.cuda.Stream()
+    other.use_stream(side)
+    other.reserve_scratch(8 << 20)
+    out = torch.empty((rows, N_HEADS, 64), device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(200_000_000)  # holds the other stream for tens of milliseconds
+    assert lib.focr_kv_attention_decode(other.handle, kv.handle, q.data_ptr(), rows, sinks.data_ptr(), out.data_ptr()) == 0
+
+    def reseal():
+        return lib.focr_kv_reseal(ctx.handle, kv.handle, k2.data_ptr(), v2.data_ptr(), P, cap)
+
+    if refused:
+        stream, graph = ctypes.c_void_p(captured.cuda_stream), ctypes.c_void_p()
+        assert lib.hipStreamBeginCapture(stream, 0) == 0  # hipStreamCaptureModeGlobal
+        rc = reseal()
+        lib.hipStreamEndCapture(stream, ctypes.byref(graph))
+        if graph:
+            lib.hipGraphDestroy(graph)
+        lib.hipGetLastError()
+        assert rc != 0
+    assert not side.query(), "the queued decode has run: nothing left to wait for"
+    assert reseal() == 0
+    torch.cuda.synchronize()
+    assert_bitwise(host(out), want, "decode over the old records")
+    for got, ref in zip(kv.dequantize()[:2], fh.KvSplit.seal(bits, k2, v2, P, cap, N_HEADS, N_KV).dequantize()[:2]):
+        assert_bitwise(host(got), host(ref), "resealed records")
+    kv.free()
+    other.close()
+
+
 @pytest.mark.parametrize("fast", [False, True])
 @pytest.mark.parametrize("bits", [8, 16])
 @pytest.mark.parametrize("prefix_len,tail,rows", [(64, 1, 1), (700, 3, 3), (2000, 8, 8), (129, 5, 2)])
