@@ -910,6 +910,28 @@ int seal_into(Ctx *ctx, KvSplit *s, const float *prefix_k, const float *v, size_
   return FOCR_OK;
 }
 
+// seal_into after focr_kv_reseal's checks and its wait for the old records'
+// readers.
+int reseal_into(Ctx *ctx, KvSplit *s, const float *prefix_k, const float *v, size_t prefix_len, size_t capacity) {
+  FOCR_REQUIRE(prefix_k && v, FOCR_E_ARG, "focr_kv_reseal: null argument");
+  FOCR_REQUIRE(prefix_len > 0 && capacity >= prefix_len && capacity < (size_t(1) << 30), FOCR_E_SHAPE,
+               "invalid split-prefix capacity");
+  FOCR_REQUIRE(prefix_len * s->n_kv * kRecord / 256 < (size_t(1) << 31), FOCR_E_SHAPE,
+               "split prefix too long for one seal launch");
+  FOCR_HIP_CHECK(hipSetDevice(ctx->device));
+  // Calls on any stream, or captured graphs, may still read the old records.
+  // A refused wait (a stream being captured) leaves them marked as in use.
+  if (s->used.exchange(false)) {
+    const hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess) {
+      s->used.store(true);
+      (void)hipGetLastError();
+      return set_error(FOCR_E_HIP, std::string("focr_kv_reseal: waiting for the old records' readers: ") + hipGetErrorString(e));
+    }
+  }
+  return seal_into(ctx, s, prefix_k, v, prefix_len, capacity);
+}
+
 }  // namespace
 }  // namespace focr
 
@@ -948,23 +970,8 @@ int focr_kv_reseal(focr_ctx *handle, focr_kv_split *kv, const float *prefix_k, c
                    size_t capacity) {
   Ctx *ctx = reinterpret_cast<Ctx *>(handle);
   KvSplit *s = reinterpret_cast<KvSplit *>(kv);
-  FOCR_REQUIRE(ctx && s && prefix_k && v, FOCR_E_ARG, "focr_kv_reseal: null argument");
-  FOCR_REQUIRE(prefix_len > 0 && capacity >= prefix_len && capacity < (size_t(1) << 30), FOCR_E_SHAPE,
-               "invalid split-prefix capacity");
-  FOCR_REQUIRE(prefix_len * s->n_kv * kRecord / 256 < (size_t(1) << 31), FOCR_E_SHAPE,
-               "split prefix too long for one seal launch");
-  FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  // Calls on any stream, or captured graphs, may still read the old records.
-  // A refused wait (a stream being captured) leaves them marked as in use.
-  if (s->used.exchange(false)) {
-    const hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess) {
-      s->used.store(true);
-      (void)hipGetLastError();
-      return set_error(FOCR_E_HIP, std::string("focr_kv_reseal: waiting for the old records' readers: ") + hipGetErrorString(e));
-    }
-  }
-  const int rc = seal_into(ctx, s, prefix_k, v, prefix_len, capacity);
+  FOCR_REQUIRE(ctx && s, FOCR_E_ARG, "focr_kv_reseal: null argument");
+  const int rc = reseal_into(ctx, s, prefix_k, v, prefix_len, capacity);
   if (rc != FOCR_OK) s->prefix_len = s->capacity = s->tail_len = 0;  // nothing to attend over or append to
   return rc;
 }

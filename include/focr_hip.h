@@ -323,8 +323,9 @@ int focr_kv_seal(focr_ctx *ctx, int bits, const float *prefix_k_dev, const float
  * and tail are dropped, its buffers are kept where they are large enough, so
  * a session's next page allocates nothing. Waits for the device if any call
  * has used the old records (a graph captured over them holds their sizes and
- * is captured again). After an error the handle holds no prefix: it is
- * resealed or freed, every other call refuses it. No reference counterpart
+ * is captured again). After any error (but a null context or handle) the
+ * handle holds no prefix: it is resealed or freed, and the calls that attend
+ * over it, decode it or append to it refuse it. No reference counterpart
  * (device state). */
 int focr_kv_reseal(focr_ctx *ctx, focr_kv_split *kv, const float *prefix_k_dev, const float *v_dev,
                    size_t prefix_len, size_t capacity);

@@ -186,6 +186,32 @@ def test_reseal_is_bitwise_a_fresh_seal(fh, bits):
     kv.free()
 
 
+@pytest.mark.parametrize("what", ["capacity", "empty", "too long", "null keys", "null values", "nonfinite"])
+def test_a_handle_whose_reseal_was_refused_holds_no_prefix(fh, what):
+    # Whatever refused it, the next calls do not answer from the old page.
+    P, cap = 70, 80
+    k, v = (to_dev(x) for x in pair_cache(P, N_KV, 85))
+    bad = v.clone()
+    bad[3, 2, 1] = float("nan")
+    one = to_dev(gen.normal((1, N_KV, 64), 1.0, 86))
+    q, sinks = to_dev(gen.normal((1, N_HEADS, 64), 1.0, 87)), to_dev(gen.uniform(N_HEADS, -2.0, 2.0, 88))
+    kv = fh.KvSplit.seal(8, k, v, P, cap, N_HEADS, N_KV)
+    kv.append(one, one, 1)
+    args = {"capacity": (k, v, P, P - 1), "empty": (k, v, 0, cap), "too long": (k, v, P, 1 << 30),
+            "null keys": (None, v, P, cap), "null values": (k, None, P, cap), "nonfinite": (k, bad, P, cap)}[what]
+    lib, ptr = fh.lib(), lambda t: None if t is None else t.data_ptr()
+    assert lib.focr_kv_reseal(kv.ctx.handle, kv.handle, ptr(args[0]), ptr(args[1]), *args[2:]) != 0
+    assert kv.info()[1:4] == (0, 0, 0)
+    for call in (lambda: kv.attention_decode(q, 1, sinks), lambda: kv.attention_decode_noalloc(q, 1, sinks, q.clone()),
+                 lambda: kv.append(one, one, 1), kv.dequantize):
+        with pytest.raises(fh.FocrError):
+            call()
+    assert lib.focr_kv_reseal(kv.ctx.handle, kv.handle, k.data_ptr(), v.data_ptr(), P, cap) == 0
+    for got, want in zip(kv.dequantize()[:2], oracle_cache(8, host(k), host(v), P, [], [], cap)):
+        assert_bitwise(host(got), want)
+    kv.free()
+
+
 @pytest.mark.parametrize("refused", [False, True])
 @pytest.mark.parametrize("bits", [8, 16])
 def test_reseal_waits_for_readers_on_other_streams(fh, bits, refused):
@@ -226,6 +252,7 @@ def test_reseal_waits_for_readers_on_other_streams(fh, bits, refused):
             lib.hipGraphDestroy(graph)
         lib.hipGetLastError()
         assert rc != 0
+        assert kv.info()[1:4] == (0, 0, 0)
     assert not side.query(), "the queued decode has run: nothing left to wait for"
     assert reseal() == 0
     torch.cuda.synchronize()
