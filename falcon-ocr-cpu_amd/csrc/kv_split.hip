@@ -91,7 +91,6 @@ struct KvSplit {
   unsigned char *records = nullptr;  // [n_kv][prefix_len][record_bytes]
   unsigned char *tail = nullptr;     // [n_kv][capacity - prefix_len][tail_bytes]
   size_t records_alloc = 0, tail_alloc = 0;  // bytes allocated, at least what the current sizes need
-  size_t device_bytes = 0;
   // Whether any call has queued work on the records since they were sealed
   // (the seal itself is synchronous): focr_kv_reseal then waits for the device.
   // Atomic: contexts may read one cache from several threads.
@@ -878,7 +877,6 @@ int seal_into(Ctx *ctx, KvSplit *s, const float *prefix_k, const float *v, size_
   hipError_t e = grow(&s->records, &s->records_alloc, rec_total);
   if (e == hipSuccess) e = grow(&s->tail, &s->tail_alloc, tail_total);
   if (e != hipSuccess) return set_error(FOCR_E_HIP, std::string("focr_kv_seal: ") + hipGetErrorString(e));
-  s->device_bytes = rec_total + tail_total;
   volatile uint32_t *flags = ctx->flags;
   flags[0] = flags[1] = flags[2] = 0;
   SealArgs a{prefix_k, v, s->records, ctx->flags, static_cast<int>(prefix_len), s->n_heads, s->n_kv,
@@ -1111,7 +1109,7 @@ int focr_kv_info(const focr_kv_split *kv, int *bits, size_t *prefix_len, size_t 
   if (prefix_len) *prefix_len = s->prefix_len;
   if (tail_len) *tail_len = s->tail_len;
   if (capacity) *capacity = s->capacity;
-  if (device_bytes) *device_bytes = s->device_bytes;
+  if (device_bytes) *device_bytes = s->records_alloc + s->tail_alloc;
   return FOCR_OK;
 }
 

@@ -403,6 +403,8 @@ int focr_kv_truncate_tail(focr_kv_split *kv, size_t tail_len);
 int focr_kv_set_fast_exp(focr_kv_split *kv, int fast);
 /* SplitPrefix::fast_exp (src/quant/kv/record_bits.rs:6-8): *fast = 0 or 1. */
 int focr_kv_fast_exp(const focr_kv_split *kv, int *fast);
+/* device_bytes: what the handle's buffers hold, those of its largest page
+ * where it was resealed with a smaller one. */
 int focr_kv_info(const focr_kv_split *kv, int *bits, size_t *prefix_len, size_t *tail_len,
                  size_t *capacity, size_t *device_bytes);
 int focr_kv_free(focr_kv_split *kv);

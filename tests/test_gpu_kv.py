@@ -145,7 +145,7 @@ def test_reseal_is_bitwise_a_fresh_seal(fh, bits):
     import torch
 
     ctx = fh.default_context()
-    kv = None
+    kv, held = None, [0, 0]
     for i, (P, cap) in enumerate([(300, 309), (37, 46), (1000, 1009), (999, 1009)]):
         k, v = pair_cache(P, N_KV, 50 + i, 2.0)
         tk, tv = gen.normal((3, N_KV, 64), 1.0, 60 + i), gen.normal((3, N_KV, 64), 1.0, 70 + i)
@@ -157,8 +157,13 @@ def test_reseal_is_bitwise_a_fresh_seal(fh, bits):
         kv.set_fast_exp(True).append(to_dev(tk), to_dev(tv), 3)
         for got, want in zip(kv.dequantize(), oracle_cache(bits, k, v, P, tk, tv, cap)):
             assert_bitwise(host(got), want)
+        # The device bytes are those the handle holds: each buffer as large as
+        # the largest page so far needed it.
         fresh = fh.KvSplit.seal(bits, kd, vd, P, cap, N_HEADS, N_KV)
-        assert kv.info() == fresh.info()[:2] + (3,) + fresh.info()[3:]
+        assert kv.info()[:4] == (bits, P, 3, cap)
+        records, tail = (N_KV * (n * bits // 8 + m) for n, m in ((160, 16), (128, 16)))
+        held = [max(held[0], P * records), max(held[1], (cap - P) * tail)]
+        assert kv.info()[4] == sum(held) and fresh.info()[4] == P * records + (cap - P) * tail
         fresh.free()
         side = torch.cuda.Stream()
         ctx.use_stream(side)
