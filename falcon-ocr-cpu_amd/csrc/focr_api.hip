@@ -20,16 +20,44 @@ int set_error(int code, const std::string &message) {
 }
 
 int ensure_scratch(Ctx *ctx, size_t bytes) {
-  if (bytes <= ctx->scratch_bytes) return FOCR_OK;
-  // Growing frees the old buffer: a graph captured earlier would replay into
-  // freed memory, and neither a free nor a synchronization may run while the
-  // stream is being captured. Callers that capture pre-grow the scratch with
-  // focr_ctx_reserve_scratch (or one uncaptured call of the same shape).
+  const bool fits = bytes <= ctx->scratch_bytes;
+  if (fits && ctx->scratch_captured) return FOCR_OK;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  FOCR_HIP_CHECK(hipStreamIsCapturing(ctx->stream, &capture));
+  const hipError_t asked = hipStreamIsCapturing(ctx->stream, &capture);
+  if (fits) {
+    // A refused query (the null stream while another stream captures) leaves
+    // no error behind for the next launch check.
+    if (asked != hipSuccess) (void)hipGetLastError();
+    ctx->scratch_captured = asked == hipSuccess && capture != hipStreamCaptureStatusNone;
+    return FOCR_OK;
+  }
+  FOCR_HIP_CHECK(asked);
+  // Neither a free nor a synchronization may run while the stream is being
+  // captured. Callers that capture pre-grow the scratch with
+  // focr_ctx_reserve_scratch (or one uncaptured call of the same shape).
   FOCR_REQUIRE(capture == hipStreamCaptureStatusNone, FOCR_E_UNSUPPORTED,
                "the context scratch must grow to " + std::to_string(bytes) +
                    " bytes, which cannot happen during stream capture; call focr_ctx_reserve_scratch first");
+  // A buffer that a captured call was given stays until the context goes: the
+  // graph replays into it. Its successor is at least twice as large, so that
+  // those kept are together smaller than the one in use.
+  if (ctx->scratch && ctx->scratch_captured) {
+    FOCR_REQUIRE(ctx->n_kept < Ctx::kKept, FOCR_E_UNSUPPORTED, "too many scratch buffers held by captured graphs");
+    void *fresh = nullptr;
+    size_t grown = std::max(bytes, 2 * ctx->scratch_bytes);
+    hipError_t err = hipMalloc(&fresh, grown);
+    if (err != hipSuccess && grown > bytes) {
+      (void)hipGetLastError();
+      grown = bytes;
+      err = hipMalloc(&fresh, grown);
+    }
+    FOCR_HIP_CHECK(err);
+    ctx->kept[ctx->n_kept++] = ctx->scratch;
+    ctx->scratch = fresh;
+    ctx->scratch_bytes = grown;
+    ctx->scratch_captured = false;
+    return FOCR_OK;
+  }
   if (ctx->scratch) {
     FOCR_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     FOCR_HIP_CHECK(hipFree(ctx->scratch));
@@ -39,6 +67,7 @@ int ensure_scratch(Ctx *ctx, size_t bytes) {
   size_t grown = std::max(bytes, static_cast<size_t>(1) << 20);
   FOCR_HIP_CHECK(hipMalloc(&ctx->scratch, grown));
   ctx->scratch_bytes = grown;
+  ctx->scratch_captured = false;
   return FOCR_OK;
 }
 
@@ -189,6 +218,7 @@ int focr_ctx_destroy(focr_ctx *handle) {
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
   FOCR_HIP_CHECK(hipStreamSynchronize(ctx->stream));
   if (ctx->scratch) FOCR_HIP_CHECK(hipFree(ctx->scratch));
+  for (int i = 0; i < ctx->n_kept; i++) FOCR_HIP_CHECK(hipFree(ctx->kept[i]));
   if (ctx->argmax) FOCR_HIP_CHECK(hipHostFree(ctx->argmax));
   if (ctx->rms_dev) FOCR_HIP_CHECK(hipFree(ctx->rms_dev));
   if (ctx->flags) FOCR_HIP_CHECK(hipHostFree(ctx->flags));

@@ -92,13 +92,15 @@ int focr_ctx_use_own_stream(focr_ctx *ctx);
 void *focr_ctx_stream(const focr_ctx *ctx);
 int focr_ctx_sync(focr_ctx *ctx);
 /* The context scratch (INT16 activation codes, attention partial states,
- * BF16 K/V copies) grows on demand by free + malloc. No reference
- * counterpart: the reference's Scratch (src/quant/linear.rs:311-315) is a
- * host Vec. Growing invalidates graphs captured earlier (they would replay
- * into freed memory) and is refused with FOCR_E_UNSUPPORTED while the
- * stream is capturing: a caller that captures reserves the largest size
- * first, or makes one uncaptured call of each shape. Synchronizes the
- * context's stream when it grows.
+ * BF16 K/V copies) grows on demand. No reference counterpart: the reference's
+ * Scratch (src/quant/linear.rs:311-315) is a host Vec. Growing is refused with
+ * FOCR_E_UNSUPPORTED while the stream is capturing: a caller that captures
+ * reserves the largest size first, or makes one uncaptured call of each shape.
+ * Graphs captured earlier stay valid when a later call grows it: a buffer that
+ * a captured call was given is kept until the context is destroyed (its
+ * successor is at least twice as large, so those kept are together smaller
+ * than the one in use); one that no capture saw is freed, after a
+ * synchronization of the context's stream.
  * Device buffers a context owns, and so the only addresses of its own that a
  * captured graph can hold: the scratch (above) and an 8-float row-scale
  * array allocated at creation (focr_argmax's result words are read back to

@@ -2,7 +2,7 @@
 scratch during capture is refused (FOCR_E_UNSUPPORTED, nothing launched);
 after focr_ctx_reserve_scratch the same call captures, and every replay of
 the graph, with eager work and synchronizations between the replays, equals
-the eager result bit for bit."""
+the eager result bit for bit, also after eager calls have grown the scratch."""
 import numpy as np
 import pytest
 
@@ -161,4 +161,56 @@ def test_fp16_pair_paths_capture_and_replay():
         assert_bitwise(host(gemm_out), gemm_eager, f"GEMM replay {rep}")
     assert ctx.scratch_bytes() == sized
     lin.free()
+    ctx.close()
+
+
+def test_a_graph_stays_valid_when_an_eager_call_grows_the_scratch():
+    # A sealed-KV decode captured over the context scratch, then eager FP32
+    # prefills that need more of it (their small grids split their keys into
+    # parts): the graph replays into the buffer it was captured with, whatever
+    # is allocated in between.
+    import torch
+
+    import focr_hip as fh
+    from test_oracle_kv import pair_cache
+
+    ctx = fh.Context(0)
+    P, rows = 3000, 2
+    k, v = (to_dev(x) for x in pair_cache(P, 8, 71, 2.0))
+    kv = fh.KvSplit.seal(8, k, v, P, P + rows, 16, 8, ctx=ctx)
+    tk, tv = to_dev(gen.normal((rows, 8, 64), 1.0, 72)), to_dev(gen.normal((rows, 8, 64), 1.0, 73))
+    kv.append(tk, tv, rows)
+    q, sinks = to_dev(gen.normal((rows, 16, 64), 1.0, 74)), to_dev(gen.uniform(16, -2.0, 2.0, 75))
+    eager = host(kv.attention_decode(q, rows, sinks))
+    sized = ctx.scratch_bytes()
+    out = torch.empty((rows, 16, 64), device="cuda:0")
+    side, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(g, stream=side):
+            ctx.use_stream(torch.cuda.current_stream())
+            kv.attention_decode(q, rows, sinks, out=out)
+    ctx.use_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    assert ctx.scratch_bytes() == sized
+    opts, held = fh.PrefillOptions(split_products=False), []
+    for L in (400, 1000, 1501):
+        pq, pk = (to_dev(gen.normal(L * 16 * 64, 1.0, 76 + i)) for i in range(2))
+        pv = to_dev(gen.normal(L * 8 * 64, 1.0, 78))
+        before = ctx.scratch_bytes()
+        cache, geom = fh.CompactKv.prefill(pk, pv, L, 16, 8), fh.Geometry(0, 0, L // 2)
+        first = host(fh.attention_with(pq, cache, L, geom, sinks, opts, ctx=ctx))
+        assert ctx.scratch_bytes() > before
+        held += [torch.full((1 << 18,), float("nan"), device="cuda:0") for _ in range(32)]
+        for rep in range(2):
+            out.fill_(float("nan"))
+            again = fh.attention_with(pq, cache, L, geom, sinks, opts, ctx=ctx)  # eager work between replays
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert_bitwise(host(out), eager, f"{L} rows, replay {rep}")
+            assert_bitwise(host(again), first, f"{L} rows, eager {rep}")
+    assert all(bool(torch.isnan(t).all()) for t in held)
+    del g
+    kv.free()
     ctx.close()
