@@ -74,7 +74,11 @@ int ensure_scratch(Ctx *ctx, size_t bytes) {
 bool scratch_fits(Ctx *ctx, size_t bytes) {
   if (bytes <= ctx->scratch_bytes) return true;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(ctx->stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess) {
+    (void)hipGetLastError();  // as in ensure_scratch; growth would be refused with it
+    return false;
+  }
+  return capture == hipStreamCaptureStatusNone;
 }
 
 // The context's work moves to a new stream only behind everything already

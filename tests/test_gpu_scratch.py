@@ -214,3 +214,37 @@ def test_a_graph_stays_valid_when_an_eager_call_grows_the_scratch():
     del g
     kv.free()
     ctx.close()
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])  # hipStreamCaptureMode Global, ThreadLocal, Relaxed
+def test_prefill_on_the_null_stream_while_a_blocking_stream_is_captured(mode):
+    # The null stream cannot be asked whether it is captured then, so the
+    # scratch does not grow and the small grid's keys are not split; the call
+    # itself runs as at any other time.
+    import ctypes
+
+    import oracle
+    import torch
+
+    import focr_hip as fh
+    from test_gpu_attention import close
+
+    ctx, lib, L, image = fh.Context(0), fh.lib(), 400, (0, 130)
+    q, k, v = gen.normal(L * 16 * 64, 1.0, 81), gen.normal(L * 16 * 64, 1.0, 82), gen.normal(L * 8 * 64, 1.0, 83)
+    sinks = gen.uniform(16, -2.0, 2.0, 84)
+    qd, kd, vd, sd, out = (to_dev(x) for x in (q, k, v, sinks, np.zeros_like(q)))
+    assert torch.cuda.current_stream().cuda_stream == 0
+    torch.cuda.synchronize()
+    stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    assert lib.hipStreamCreate(ctypes.byref(stream)) == 0 and lib.hipStreamBeginCapture(stream, mode) == 0
+    try:
+        fh.attention_with(qd, fh.CompactKv.prefill(kd, vd, L, 16, 8), L, fh.Geometry(0, *image), sd,
+                          fh.PrefillOptions(split_products=False), output=out, ctx=ctx)
+    finally:
+        assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+        lib.hipGraphDestroy(graph)
+        lib.hipStreamDestroy(stream)
+    torch.cuda.synchronize()
+    assert ctx.scratch_bytes() == 0
+    close(host(out).reshape(L, 16, 64), oracle.attention_prefill(q, k, v, L, L, L, 16, 8, 0, *image, sinks))
+    ctx.close()
