@@ -1385,12 +1385,17 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
   // By 32 x 32 blocks of output (us, this form and its neighbours): 120 (WO,
   // m = 144) 32 x 32 5.7, 32 x 64 7.0; 288 (W13, 48) 32 x 64 6.5, 32 x 32 8.0;
   // 312 (W2, 400) 32 x 64 13.9, 32 x 32 16.4, 64 x 64 18.3; 528 (W2, 700) 64 x 64
-  // 18.8, 32 x 64 22+; 1,872 (W13, 400) 64 x 64 17.2, split_kernel 17.7; 3,000
-  // (WO, 4,000) 29.1 and 30.3; 3,008 (QKV, 1,501) 24.2 and 24.0; 3,168 (W13, 700)
-  // 29.4 and 24.2.
+  // 18.8, 32 x 64 22+.
+  // The 64 x 64 form reads its operands once a wave: it gains up to one
+  // workgroup per compute unit (1,024 blocks), and past that, where the launch
+  // and epilogue count for less, from a k of 2,048 on. us per call, operand
+  // planes included, 64 x 64 form / split_kernel's 64-row tiles, n = 768: 984
+  // blocks k = 192 10.9 / 11.0, 768 15.2 / 18.9, 2,304 29.0 / 43.2; 1,200 blocks
+  // k = 256 12.5 / 11.3, 768 20.3 / 18.8, 2,304 42.4 / 43.1; 2,184 blocks (2,912
+  // rows) k = 1,024 34.3 / 31.3, 2,304 59.7 / 58.7, 4,096 99.7 / 100.4.
   auto launch_small = [&](auto ib, auto jb, auto wk, auto depth) {
     constexpr int IB = decltype(ib)::value, JB = decltype(jb)::value, WK = decltype(wk)::value, D = decltype(depth)::value;
-    const int rt = static_cast<int>((rows + 32 * IB - 1) / (32 * IB)), ct = static_cast<int>(n_pad / (32 * JB));
+    const int rt = static_cast<int>((rows + 32 * IB - 1) / (32 * IB)), ct = static_cast<int>((lin->n + 32 * JB - 1) / (32 * JB));
     const dim3 grid(static_cast<unsigned>(rt * ct));
     if (epilogue == FOCR_EPI_GLU)
       hipLaunchKernelGGL((split_small_kernel<FOCR_EPI_GLU, IB, JB, WK, D>), grid, dim3(64 * WK), 0, ctx->stream, a, ap, bp,
@@ -1404,7 +1409,7 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
   };
   using std::integral_constant;
   const size_t blocks = ((rows + 31) / 32) * ((lin->n + 31) / 32);
-  if (blocks <= 3000) {
+  if (blocks <= 420 || (k32 >= 192 && blocks <= 1024) || (k32 >= 2048 && blocks <= 3000)) {
     if (blocks <= 160)
       launch_small(integral_constant<int, 1>(), integral_constant<int, 1>(), integral_constant<int, 8>(),
                    integral_constant<int, 4>());
