@@ -1424,10 +1424,13 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
   }
   // 256- and 128-row tiles fill 512 workgroup slots (two per compute unit, by
   // VGPRs). 256-row tiles take whole rounds, and all rows where the last round
-  // is at least 0.3 full behind a whole one or 0.8 full as the only one; the
-  // rows left (or all of them) run as 128-row tiles, or as 64-row tiles (twice
-  // as many, half the work each) where those would fill less than 0.8 of their
-  // only round, or at most half of their last one.
+  // is at least 0.3 full behind a whole one or 0.8 full as the only one and no
+  // odd 128 rows are left over: a launch of its own that walks all of k for one
+  // row of tiles. (n = 768, 20,000 rows of k = 768: 98 without 256-row tiles, 109
+  // with them and the odd row; W13, 3,200 rows 79 and 87, 6,000 rows 144 and 150.)
+  // The rows left (or all of them) run as 128-row tiles, or as 64-row tiles
+  // (twice as many, half the work each) where those would fill less than 0.8 of
+  // their only round, or at most half of their last one.
   // us per call, 128- and 64-row tiles alone -> with 256-row tiles: QKV 6,544
   // (0.81 rounds) 82 -> 79, 16,320 (2.0) 188 -> 175; W13 6,544 (1.83) 169 -> 158,
   // 12,000 (3.30) 284 -> 261 (267 with only the whole rounds), 16,320 372 -> 349;
@@ -1440,7 +1443,7 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
   const integral_constant<int, 128> mid;
   const integral_constant<int, 64> low;
   const int tall_tiles = rt128 / 2 * ctiles, tall_left = tall_tiles % kSlots;
-  const bool all_tall = 10 * tall_left >= (tall_tiles > kSlots ? 3 : 8) * kSlots;
+  const bool all_tall = rt128 % 2 == 0 && 10 * tall_left >= (tall_tiles > kSlots ? 3 : 8) * kSlots;
   const int tall_rows = all_tall ? rt128 / 2 : (tall_tiles - tall_left) / ctiles;
   if (tall_rows > 0) launch(tall, 0, tall_rows);
   const int first = 2 * tall_rows, rest = rt128 - first;  // 128-row tiles

@@ -254,9 +254,11 @@ def test_f32_split_tile_heights(fh, m):
 # rows), one whole round and an odd 128 rows (4,200), whole rounds with the
 # rest as 64-row tiles (5,000) and as 128-row ones (2,900 of 8,192), every row
 # behind a whole round (6,600); and a round of 128-row tiles 0.83 full (9,000
-# of 768). Stage counts around the ring's length.
+# of 768). Odd numbers of 128-row tiles where 256-row ones would be alone in a
+# round 0.81 full (3,400: none of them) and behind a whole round (6,300: one round
+# of them, the rest as 128-row tiles). Stage counts around the ring's length.
 @pytest.mark.parametrize("m,k,n", [(3300, 64, 4096), (4200, 32, 4090), (5000, 160, 4096), (2900, 64, 8192), (6600, 96, 4096),
-                                   (9000, 64, 768)])
+                                   (9000, 64, 768), (3400, 96, 4096), (6300, 64, 4096)])
 def test_f32_split_tall_tiles(fh, m, k, n):
     oracle.set_threads(oracle_threads())
     a, w = gen.normal((m, k), 1.0, 47), gen.normal((n, k), 0.02, 48)
