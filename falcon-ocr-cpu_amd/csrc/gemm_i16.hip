@@ -491,11 +491,17 @@ int launch_prefill_i16(Ctx *ctx, const Linear *lin, const float *x, size_t rows,
   // and its neighbours, quantizer not counted): 432 (WO, m = 144) 16 x 16 per wave
   // 4.5, 16 x 32 5.8, gemm_kernel 10; 864 (W13, 48) 4.4, 5.0; 2,592 (W13, 144)
   // 16 x 32 7.1, 16 x 16 8.4, 32 x 32 8.4, gemm_kernel 9.7; 3,024 (W2, 1,000) 14.5,
-  // 18.5, 18.2, 20; 4,512 (W2, 1,501) 32 x 32 20.5, 16 x 32 21.0, gemm_kernel 23;
-  // 7,200 (W13, 400) 32 x 32 11.9, gemm_kernel 13.8; 7,536 (W2, 2,500) 24.9 and
-  // 23.4; 8,064 (QKV, 1,000) 12.3 and 11.3: larger grids share operands in LDS.
+  // 18.5, 18.2, 20. Larger grids share operands in LDS (gemm_kernel): from 4,000
+  // blocks on where its tiles are 64 columns wide (us per call, 32 x 32 here and
+  // gemm_kernel: W2, 1,664 rows 28.1 and 28.4, 2,432 32.7 and 29.6; k = 8,192, 2,432
+  // rows 102 and 84); where they are 128 wide, from 5,500 on (W13, 320 rows 13.6 and
+  // 13.9, 384 14.7 and 13.3; a k below 768 from 4,000 on: 256 -> 3,072, 304 rows 7 %
+  // slower here), but not before 7,400 where its grid, padded to 128 rows, starts a
+  // second round of one workgroup per compute unit (W13, 400 rows 14.9 and 16.1).
   const size_t blocks = (m + 15) / 16 * (n / 16);
-  if (blocks <= 7400) {
+  const bool wide = n >= 2048;  // gemm_kernel's tiles are 128 columns wide
+  const size_t wide_tiles = m_pad / kBM * ((n + 127) / 128);
+  if (blocks <= 4000 || (wide && ((blocks <= 5500 && k >= 768) || (blocks <= 7400 && wide_tiles > 256)))) {
     auto launch = [&](auto epi, auto rb, auto cb, auto wv, auto depth) {
       constexpr int E = decltype(epi)::value, RB = decltype(rb)::value, CB = decltype(cb)::value;
       constexpr int WV = decltype(wv)::value, D = decltype(depth)::value;
@@ -537,7 +543,6 @@ int launch_prefill_i16(Ctx *ctx, const Linear *lin, const float *x, size_t rows,
                      lin->exc_vals, static_cast<int>(lin->n_exc), static_cast<int>(m), static_cast<int>(n),          \
                      static_cast<int>(groups), static_cast<int>(row_blocks), static_cast<int>(m_pad), row_tiles,     \
                      static_cast<int>((n + BN - 1) / BN), out)
-  const bool wide = n >= 2048;
   if (epilogue == FOCR_EPI_GLU) {
     if (wide) FOCR_LAUNCH_I16(FOCR_EPI_GLU, 128); else FOCR_LAUNCH_I16(FOCR_EPI_GLU, 64);
   } else if (epilogue == FOCR_EPI_ADD) {

@@ -45,9 +45,10 @@ def test_i16_panels_bitwise_every_epilogue(fh, m, k, n):
 
 # The small-grid forms (16 x 16, 16 x 32 and 32 x 32 outputs per wave by the
 # number of 16 x 16 blocks) and the LDS tiles above them, 64 and 128 columns
-# wide, with ragged rows and odd column-block counts.
+# wide, with ragged rows and odd column-block counts; both sides of their lines.
 @pytest.mark.parametrize("m,k,n", [(9, 64, 32), (33, 320, 1056), (130, 192, 2208), (301, 256, 4128), (2500, 128, 800),
-                                   (1010, 192, 2080)])
+                                   (1010, 192, 2080), (1270, 64, 800), (1290, 64, 800), (330, 768, 4128), (340, 768, 4128),
+                                   (396, 64, 4608), (410, 64, 4608), (410, 128, 4704)])
 def test_i16_tile_forms_are_bitwise_the_panels(fh, m, k, n):
     test_i16_panels_bitwise_every_epilogue(fh, m, k, n)
 
