@@ -46,9 +46,8 @@ struct Ctx {
   // Scratch owned by the context, grown on demand (INT16 activation codes).
   void *scratch = nullptr;
   size_t scratch_bytes = 0;
-  bool scratch_captured = false;  // a call being captured was given the scratch
   static constexpr int kKept = 48;  // 1 MB doubled more often than the card's memory allows
-  void *kept[kKept] = {};           // earlier scratch buffers that captured graphs may hold
+  void *kept[kKept] = {};           // scratch buffers outgrown: captured graphs may hold them
   int n_kept = 0;
   ArgmaxPart *argmax = nullptr;  // focr_argmax's results, pinned host memory
   size_t argmax_parts = 0;
@@ -57,9 +56,8 @@ struct Ctx {
   hipEvent_t order = nullptr;  // orders a new stream after the old one (focr_ctx_set_stream)
 };
 
-// Grows the context scratch to at least `bytes` (hipMalloc on growth only) for
-// the call that is being made; a buffer given to a captured call outlives its
-// successors.
+// Grows the context scratch to at least `bytes` (hipMalloc on growth only). The
+// buffers it outgrows live as long as the context.
 int ensure_scratch(Ctx *ctx, size_t bytes);
 // Whether ensure_scratch(ctx, bytes) can succeed now: it cannot grow while the
 // stream is being captured.

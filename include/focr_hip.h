@@ -97,10 +97,9 @@ int focr_ctx_sync(focr_ctx *ctx);
  * FOCR_E_UNSUPPORTED while the stream is capturing: a caller that captures
  * reserves the largest size first, or makes one uncaptured call of each shape.
  * Graphs captured earlier stay valid when a later call grows it: a buffer that
- * a captured call was given is kept until the context is destroyed (its
- * successor is at least twice as large, so those kept are together smaller
- * than the one in use); one that no capture saw is freed, after a
- * synchronization of the context's stream.
+ * it outgrows is kept until the context is destroyed (its successor is at
+ * least twice as large, so those kept are together smaller than the one in
+ * use).
  * Device buffers a context owns, and so the only addresses of its own that a
  * captured graph can hold: the scratch (above) and an 8-float row-scale
  * array allocated at creation (focr_argmax's result words are read back to
