@@ -215,15 +215,18 @@ void launch_tile(const GemmArgs &a, hipStream_t stream) {
 // 23.2; 3,200 (QKV, 400) 32 x 64 22.8, 64 x 64 24.2; 4,512 (WO, 1,501) 32 x 64
 // 37.8, 64 x 64 44.6; 8,064 (QKV, 1,000) 64 x 64 38.0, 32 x 64 43.5; 27,072
 // (W13, 1,501) 64 x 64 121, 64 x 128 132; 45,216 (W13, 2,500) 64 x 128 195,
-// 64 x 64 202.
+// 64 x 64 202. FP32 weights of k = 64, one or two stages, go on to the next form
+// earlier: 150 x 64 -> 4,096 (2,560 blocks) 16 x 64 8.8, 32 x 64 6.6; 300 rows
+// (4,864) 32 x 64 9.5, 64 x 64 6.5.
 template <typename T, int EPI>
 void launch_epilogue(const GemmArgs &a, hipStream_t stream) {
   const long blocks = static_cast<long>((a.m + 15) / 16) * ((a.n + 15) / 16);
+  const bool brief = std::is_same<T, float>::value && a.k == 64;
   if (blocks <= 1280)
     launch_tile<T, EPI, 1, 2, 1, 1, 64, 4>(a, stream);
-  else if (blocks <= 3100)
+  else if (blocks <= (brief ? 2000 : 3100))
     launch_tile<T, EPI, 1, 4, 1, 1, 64, 4>(a, stream);
-  else if (blocks <= 5500)
+  else if (blocks <= (brief ? 4000 : 5500))
     launch_tile<T, EPI, 2, 2, 1, 2, 64, 3>(a, stream);
   else if (blocks <= 36000)
     launch_tile<T, EPI, 2, 2, 2, 2, 32, 3>(a, stream);
@@ -246,11 +249,15 @@ void launch_type(const GemmArgs &a, int epilogue, hipStream_t stream) {
 // Whole 64-wide k stages (one scale group per stage for codes), 16-byte
 // aligned rows, no exception columns (their values would have to replace the
 // codes in k order), 32-bit offsets within a tile, and a grid whose tile
-// count an int holds.
+// count an int holds. FP32 weights of k = 64 past 12,500 blocks keep chain2's
+// tiles, which do not repeat a ring of copies for two stages of work (us per
+// call, here and there: 6,544 x 64 -> 4,096 67 and 56, 992 x 64 -> 2,048 7.0 and
+// 9.2; at k = 128 39 and 44 for 2,400 rows; codes are faster here at any k).
 bool launch_chain_mfma(const GemmArgs &a, int bits, int epilogue, hipStream_t stream) {
   const bool aligned = (reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.codes)) % 16 == 0;
   if (!aligned || a.k % 64 != 0 || a.k > (1 << 20) || a.n_exc != 0 || (bits != 32 && a.group % 64 != 0)) return false;
-  if (static_cast<long>((a.m + 15) / 16) * ((a.n + 15) / 16) >= (long(1) << 31)) return false;
+  const long blocks = static_cast<long>((a.m + 15) / 16) * ((a.n + 15) / 16);
+  if (blocks >= (long(1) << 31) || (bits == 32 && a.k == 64 && blocks > 12500)) return false;
   if (bits == 8)
     launch_type<int8_t>(a, epilogue, stream);
   else if (bits == 16)

@@ -767,8 +767,8 @@ void launch_one(bool chain, const GemmArgs &a, hipStream_t stream) {
     if (a.k % kC2K == 0 && aligned && (std::is_same<T, float>::value || a.group % 8 == 0)) {
       // 128 x 128 tiles where they give at least two per compute unit,
       // 64 x 64 ones otherwise (n = 768 at 6,544 rows: WO 0.264 -> 0.195 ms).
-      // Only exception columns, k not a multiple of 64 and groups of 32
-      // reach these.
+      // Only exception columns, k not a multiple of 64, groups of 32 and FP32
+      // weights of k = 64 reach these.
       const long big = static_cast<long>((a.m + 127) / 128) * ((a.n + 127) / 128);
       if (big >= 512)
         hipLaunchKernelGGL((chain2_kernel<T, EPI, 128, 128>), dim3((a.m + 127) / 128, (a.n + 127) / 128), dim3(256), 0,

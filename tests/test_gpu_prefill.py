@@ -142,10 +142,12 @@ def test_f32_chain_is_bitwise_the_panels(fh, bits, m, k, n):
 
 # One shape per tile form of the matrix-core chain (16 x 32, 16 x 64, 32 x 64,
 # 64 x 64 and 64 x 128 outputs, chosen by the number of 16 x 16 blocks), each
-# with ragged rows and columns and with stage counts around the ring's length.
+# with ragged rows and columns and with stage counts around the ring's length;
+# k = 64 either side of 12,500 blocks, past which FP32 weights take the SIMT tiles.
 @pytest.mark.parametrize("bits", [32, 16, 8])
 @pytest.mark.parametrize("m,k,n", [(17, 64, 50), (33, 320, 1298), (150, 128, 2500), (300, 192, 3210), (515, 320, 4098),
-                                   (2070, 64, 4500)])
+                                   (2070, 64, 4500), (2070, 128, 4500), (260, 64, 2010), (300, 64, 3500),
+                                   (720, 64, 4390), (720, 64, 4470)])
 def test_f32_chain_tile_forms_are_bitwise_the_panels(fh, bits, m, k, n):
     test_f32_chain_is_bitwise_the_panels(fh, bits, m, k, n)
 
