@@ -893,12 +893,12 @@ int launch_tiles(Ctx *ctx, AttnArgs a, int softmax, int exp_mode) {
   split::Plan plan;
   int slots = 0;
   int items = split::make_plan(plan, tiles, a.query_len, a.query_offset, a.image_start, a.image_end, a.n_heads, kKeys,
-                               split::kSplitItemsF32, true, &slots);
+                               split::kSplitItemsF32, &split::kSmallF32, &slots);
   // A captured call whose reserved scratch the small-grid split outgrows
   // runs without it.
   if (slots > 0 && !scratch_fits(ctx, static_cast<size_t>(slots) * a.n_heads * kQueries * 66 * sizeof(float)))
     items = split::make_plan(plan, tiles, a.query_len, a.query_offset, a.image_start, a.image_end, a.n_heads, kKeys,
-                             split::kSplitItemsF32, false, &slots);
+                             split::kSplitItemsF32, nullptr, &slots);
   a.tiles = tiles;
   a.slots = slots;
   a.part = nullptr;
@@ -1026,12 +1026,12 @@ int launch_attention_split(Ctx *ctx, const float *q, const float *k, const float
     split::Plan plan;
     int slots = 0;
     int items = split::make_plan(plan, tiles, n, static_cast<int>(q0), a.image_start, a.image_end, a.n_heads, kKeys,
-                                 split::kSplitItemsPair, true, &slots);
+                                 split::kSplitItemsPair, &split::kSmallPair, &slots);
     // A captured call whose reserved scratch the small-grid split outgrows
     // runs without it.
     if (slots > 0 && !scratch_fits(ctx, kv_bytes + static_cast<size_t>(slots) * n_heads * kQueries * 66 * sizeof(float)))
       items = split::make_plan(plan, tiles, n, static_cast<int>(q0), a.image_start, a.image_end, a.n_heads, kKeys,
-                               split::kSplitItemsPair, false, &slots);
+                               split::kSplitItemsPair, nullptr, &slots);
     a.q = q + q0 * n_heads * 64;
     a.out = out + q0 * n_heads * 64;
     a.query_len = n;

@@ -580,7 +580,7 @@ int launch_attention_bf16(Ctx *ctx, const float *q, const float *k, const float 
     split::Plan plan;
     int slots = 0;
     const int items = split::make_plan(plan, qtiles, n, static_cast<int>(q0), a.image_start, a.image_end,
-                                       a.n_heads, 128, split::kSplitItemsBf16, false, &slots);
+                                       a.n_heads, 128, split::kSplitItemsBf16, nullptr, &slots);
     a.q_base = static_cast<int>(q0);
     a.qtiles = qtiles;
     a.slots = slots;

@@ -3,9 +3,9 @@
 // A 128-query tile of a causal or image-prefixed prefill sees between 128 and
 // the whole context's keys, so one workgroup per tile leaves the chip idle
 // while the last (longest) tiles finish. Each tile's visible keys are split
-// into equal work items (about `target_items` items per call, at least
-// kMinChunkKeys keys each); an item runs the tile's online softmax over its keys only and,
-// when its tile is split, stores the unnormalized state (max, denominator,
+// into equal work items (about `target_items` items per call, of about
+// kMinChunkKeys keys or more; of kSmallChunkKeys or more in small grids); an item
+// runs the tile's online softmax over its keys only and, when its tile is split, stores the unnormalized state (max, denominator,
 // output) per query row. merge_kernel combines the parts of a row in part
 // order — M = max of the maxima, den = sum den_p exp(m_p - M),
 // o = sum o_p exp(m_p - M) — and applies the final step of
@@ -31,16 +31,31 @@ constexpr long long kSplitItemsBf16 = 1536;
 constexpr long long kSplitItemsPair = 3072;
 constexpr long long kMinChunkKeys = 1024;
 // With at most one workgroup per compute unit (tiles x heads), the FP32 and
-// FP16-pair kernels are bound by the chain of one workgroup's key tiles (1.35
-// us each with one wave per SIMD): such calls take parts of down to 192 keys,
-// about two workgroups per compute unit. FP16-pair prefill, 16 heads, us: 225
-// rows 27.7 -> 25.8, 400 34 -> 29, 700 48 -> 36, 1,000 64 -> 42, 1,501 66 ->
-// 55, 2,000 77 -> 75; at 2,500 rows (320 workgroups) 96 -> 102, and at 144
-// rows two parts and their merge 22.4 -> 24.3, so neither is split further.
-// (The BF16 kernel's tiles are too short for it: 1,000 rows 26.7 -> 25.0, 400
-// rows 15.2 -> 15.6.)
-constexpr int kSmallGrid = 256;
+// FP16-pair kernels are bound by the chain of one workgroup's key tiles (1.2 us
+// per 32 keys with one wave per SIMD in the FP16-pair kernel, 2.4 us in the FP32
+// one): such calls take parts of about 192 keys or more, about two workgroups per
+// compute unit, where that is estimated to be faster than the plan above it.
+// The estimate, in keys: the longest item, times the items a compute unit holds
+// and how far they run beside each other, plus the merge. Two workgroups of the
+// FP16-pair kernel overlap fully; those of the FP32 kernel, bound by the matrix
+// cores, hardly, and run in whole rounds. The constants are fitted to 1,790
+// measured plans of 1 to 256 heads and 9 to 16,900 visible keys: the rule loses
+// at most 4 % (FP16 pairs) and 8 % (FP32) against either plan, 0.1 % on average.
+// us per call, without / with the small parts. FP16 pairs, 16 heads, 0.6 of the
+// rows an image: 225 rows 27.5 / 25.2, 400 34.1 / 30.0, 1,000 63 / 42, 1,501 66 /
+// 55; 64 heads, 314 rows 37.0 and 37.5 (not split). FP32, 16 heads: 512 rows 47 /
+// 25, 1,024 91 / 57, 2,000 rows of 1,600 image 158 and 180 (not split); 128 heads,
+// 256 rows 30 and 36 (not split). The BF16 kernel's tiles are too short for
+// it: 1,000 rows 26.7 -> 25.0, 400 rows 15.2 -> 15.6.
+constexpr int kComputeUnits = 256;
 constexpr long long kSmallItems = 512, kSmallChunkKeys = 192;
+struct SmallGrid {
+  double share;        // of an item's time that each one on a shared compute unit takes
+  bool rounds;         // items count in whole rounds of one per compute unit
+  double merge, slot;  // the merge as such, and per partial state and head
+};
+constexpr SmallGrid kSmallPair = {0.5, false, 40.0, 0.3};
+constexpr SmallGrid kSmallF32 = {0.85, true, 60.0, 0.05};
 
 // Work plan (computed on the host, passed by value): query tiles in dispatch
 // order i (tile tiles - 1 - i: the latest, longest tiles first), each split
@@ -69,10 +84,43 @@ __host__ __device__ inline int tile_visible_end(int tile, int query_len, int que
   return intersects ? (last_abs + 1 > image_end ? last_abs + 1 : image_end) : last_abs + 1;
 }
 
+// Keys per part of a tile of `end` visible keys cut into parts of at most
+// `chunk` keys, as equal as multiples of `align` allow.
+inline int part_keys(int end, long long chunk, int align) {
+  const int parts = static_cast<int>((end + chunk - 1) / chunk);
+  return ((end + parts - 1) / parts + align - 1) / align * align;
+}
+
+// The items of tiles of vis[] keys cut into parts of at most `chunk`.
+struct Cut {
+  long long items = 0, slots = 0;
+  int part = 0, whole = 0;  // the longest part of a split tile, the longest unsplit tile
+};
+inline Cut cut_of(const int *vis, int tiles, long long chunk, int align) {
+  Cut c;
+  for (int t = 0; t < tiles; t++) {
+    const int per = part_keys(vis[t], chunk, align), parts = (vis[t] + per - 1) / per;
+    int &longest = parts > 1 ? c.part : c.whole;
+    const int keys = parts > 1 ? per : vis[t];
+    longest = keys > longest ? keys : longest;
+    c.items += parts;
+    c.slots += parts > 1 ? parts : 0;
+  }
+  return c;
+}
+inline double estimate(const Cut &c, int n_heads, const SmallGrid &g) {
+  const long long items = c.items * n_heads;
+  const double full = g.rounds ? static_cast<double>((items + kComputeUnits - 1) / kComputeUnits)
+                               : static_cast<double>(items) / kComputeUnits;
+  const double share = items <= kComputeUnits || full * g.share < 1.0 ? 1.0 : full * g.share;
+  return (c.part > c.whole ? c.part : c.whole) * share + (c.slots > 0 ? g.merge + g.slot * c.slots * n_heads : 0.0);
+}
+
 // Builds the plan for `tiles` (<= kMaxTiles) tiles; part sizes are multiples
-// of `align` keys. Returns the number of work items; *slots = partial slots.
+// of `align` keys. `small` (optional): the small-grid parts may be taken.
+// Returns the number of work items; *slots = partial slots.
 inline int make_plan(Plan &plan, int tiles, int query_len, int query_offset, int image_start, int image_end,
-                     int n_heads, int align, long long target_items, bool small_grid, int *slots_out) {
+                     int n_heads, int align, long long target_items, const SmallGrid *small, int *slots_out) {
   long long total = 0;
   int vis[kMaxTiles], most = 0;
   for (int t = 0; t < tiles; t++) {
@@ -85,16 +133,23 @@ inline int make_plan(Plan &plan, int tiles, int query_len, int query_offset, int
   // Tiles of nearly equal cost (an all-image or short prefill) balance by
   // themselves: splitting them would only add the merge traffic.
   if (5LL * most <= 6LL * total / (tiles > 0 ? tiles : 1)) chunk = most;
-  if (small_grid && static_cast<long long>(tiles) * n_heads <= kSmallGrid) {
+  if (small && static_cast<long long>(tiles) * n_heads <= kComputeUnits) {
     const long long few = total * static_cast<long long>(n_heads) / kSmallItems;
-    const long long small = ((few > kSmallChunkKeys ? few : kSmallChunkKeys) + align - 1) / align * align;
-    chunk = small < chunk ? small : chunk;
+    long long fine = ((few > kSmallChunkKeys ? few : kSmallChunkKeys) + align - 1) / align * align;
+    fine = fine < chunk ? fine : chunk;
+    Cut c = cut_of(vis, tiles, fine, align);
+    // An unsplit tile longer than the parts would be the longest item: it is
+    // cut too (256 rows of 153 image, 28.7 -> 25.4 us).
+    if (c.part > 0 && c.whole > c.part) {
+      fine = c.part;
+      c = cut_of(vis, tiles, fine, align);
+    }
+    if (estimate(c, n_heads, *small) < estimate(cut_of(vis, tiles, chunk, align), n_heads, *small)) chunk = fine;
   }
   int items = 0, slots = 0;
   for (int i = 0; i < tiles; i++) {
     const int end = vis[tiles - 1 - i];
-    const int want_parts = static_cast<int>((end + chunk - 1) / chunk);
-    const int per = ((end + want_parts - 1) / want_parts + align - 1) / align * align;
+    const int per = part_keys(end, chunk, align);
     const int parts = (end + per - 1) / per;  // every part starts before `end`
     plan.first[i] = items;
     plan.slot[i] = parts > 1 ? slots : -1;

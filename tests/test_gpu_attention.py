@@ -140,13 +140,15 @@ def norm8(n_heads, rows, seed):
     return (x * (8.0 / np.linalg.norm(x, axis=-1, keepdims=True))).astype(np.float32)
 
 
-# Small grids split their tiles' keys into parts of down to 192 keys: around
-# the first split, where the last tile is one row, the last small grid (2,048
-# rows of 16 heads) and the first that is not one.
+# Small grids may split their tiles' keys into parts of about 192 keys or more:
+# around the first split, where the last tile is one row, an image tile that is
+# only cut because it is longer than the parts (153 of 256), plans that are
+# refused (1,800 rows in the FP32 kernel), the last small grid (2,048 rows of 16
+# heads) and the first that is not one.
 @pytest.mark.parametrize("static", [False, True])
 @pytest.mark.parametrize("products", ["split", "fp32"])
-@pytest.mark.parametrize("L,image", [(192, (0, 100)), (193, (0, 193)), (385, (3, 200)), (1030, (0, 600)), (2048, (0, 1300)),
-                                     (2049, (0, 1300))])
+@pytest.mark.parametrize("L,image", [(192, (0, 100)), (193, (0, 193)), (256, (0, 153)), (385, (3, 200)), (1030, (0, 600)),
+                                     (1800, (0, 1440)), (2048, (0, 1300)), (2049, (0, 1300))])
 def test_small_grids_split_their_keys(fh, L, image, products, static):
     oracle.set_threads(8)
     q, k, v = norm8(16, L, 401).reshape(-1), norm8(16, L, 402).reshape(-1), gen.normal(L * 8 * 64, 1.0, 403)
