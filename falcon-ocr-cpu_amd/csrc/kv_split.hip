@@ -577,6 +577,31 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
         qv[r][4 * i + 3] = t.w;
       }
   }
+  // The scores are dots with the codes, which are up to 2^15 larger than the
+  // values in units of the step: where a query of these rows is past 2^100 they
+  // are scaled down by 2^64 (exactly) so that the dots stay in range, and the
+  // scores back up. Each lane looks at two of a row's 128 values. Calls of one
+  // or two rows, a step's usual ones, do not look (0.25 us of 8 us at 300
+  // positions): their queries are to stay below 2^107.
+  bool huge = false;
+  if (M > 1 && rows > 2) {
+    bool past = false;
+#pragma unroll
+    for (int r = 0; r < M; r++) {
+      const int row = row0 + r < rows ? row0 + r : rows - 1;
+      const float2 t =
+          *reinterpret_cast<const float2 *>(a.q + (static_cast<size_t>(row) * a.n_heads + 2 * g) * 64 + 2 * lane);
+      past |= __builtin_fmaxf(fabsf(t.x), fabsf(t.y)) > 1.2676506e30f;
+    }
+    huge = __any(past);
+  }
+  const float unit = huge ? 2305843009213693952.0f : 0.125f;  // 2^61 or 2^-3
+  if (huge) {
+#pragma unroll
+    for (int r = 0; r < M; r++)
+#pragma unroll
+      for (int i = 0; i < 32; i++) qv[r][i] *= 5.421010862427522e-20f;  // 2^-64
+  }
   const float ninf = -__builtin_inff();
   float m[M], dl[M];
   float4 o[M][2];
@@ -627,7 +652,7 @@ __global__ __launch_bounds__(256) void split_scan_kernel(SplitDecArgs a, int ite
     for (int r = 0; r < M; r++) {
       const float part = acc[r] * kstep;
       const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(part), __float_as_uint(part), false, false);
-      float sc = (__uint_as_float(sw[0]) + __uint_as_float(sw[1])) * 0.125f;
+      float sc = (__uint_as_float(sw[0]) + __uint_as_float(sw[1])) * unit;
       sc = j < vis[r] ? sc : ninf;
       // Slice maximum over the 16 keys (every lane of the row gets it).
       float bm = sc;

@@ -366,8 +366,10 @@ int focr_kv_decode_row(focr_ctx *ctx, focr_kv_split *kv, const float *qkv_dev, c
  * 568-580,856-900): q_dev [rows][n_heads][64], rows 1..8 (at most the
  * appended positions); row r attends to keys [0, len - rows + r + 1) of the
  * len cached positions, with the per-head sink; out_dev [rows][n_heads][64].
- * Within FP32 rounding of the compact kernel over the decoded values. Uses
- * the context scratch for the partial states. */
+ * Within FP32 rounding of the compact kernel over the decoded values (one or
+ * two rows: for queries below 2^107 in magnitude, past which their dots with
+ * the codes leave FP32's range; rotated queries are at most 8). Uses the
+ * context scratch for the partial states. */
 int focr_kv_attention_decode(focr_ctx *ctx, const focr_kv_split *kv, const float *q_dev, size_t rows,
                              const float *sinks_dev, float *out_dev);
 /* focr_kv_attention_decode with its partial softmax states in a fixed

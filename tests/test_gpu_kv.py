@@ -294,6 +294,29 @@ def test_decode_within_fp32_rounding_of_the_compact_oracle(fh, bits, prefix_len,
     kv.free()
 
 
+@pytest.mark.parametrize("bits", [8, 16])
+@pytest.mark.parametrize("rows", [3, 4, 5, 8])
+def test_huge_queries_over_tiny_keys_give_ordinary_scores(fh, bits, rows):
+    # Queries of 1e34 times keys of 1e-34: every product and score is ordinary,
+    # but a query times a code is not (32,767 x 1e34). One and two rows take
+    # queries below 2^107 only.
+    P, tail = 500, 8
+    k, v = pair_cache(P, N_KV, 97)
+    k = (k * F32(1e-34)).astype(F32)
+    tk, tv = gen.normal((tail, N_KV, 64), 1e-34, 98), gen.normal((tail, N_KV, 64), 1.0, 99)
+    q = gen.normal((rows, N_HEADS, 64), 1.0, 100)
+    q[:, 1::2] *= F32(1e34)  # one head of each pair; the other one's scores are all tiny
+    sinks = gen.uniform(N_HEADS, -2.0, 2.0, 101)
+    kv = fh.KvSplit.seal(bits, to_dev(k), to_dev(v), P, P + tail, N_HEADS, N_KV)
+    kv.append(to_dev(tk), to_dev(tv), tail)
+    got = host(kv.attention_decode(to_dev(q), rows, to_dev(sinks)))
+    pk, vals, gk = oracle_cache(bits, k, v, P, tk, tv, P + tail)
+    want = oracle.attention_decode(q, pk, gk, vals, rows, P, P + tail, N_HEADS, N_KV, P + tail - rows, 0, 0, sinks)
+    assert np.all(np.isfinite(want)) and np.all(np.isfinite(got))
+    assert np.all(np.abs(got - want) <= 1e-5 * (1 + np.abs(want)))
+    kv.free()
+
+
 def test_config5_decode_over_q8_records(fh):
     # BASELINE config 5's decode: a 16,320-row prefix, 64 generated
     # positions, one query row at 16,384 (sampled against the oracle), with
