@@ -270,7 +270,10 @@ def test_reseal_waits_for_readers_on_other_streams(fh, bits, refused):
 
 @pytest.mark.parametrize("fast", [False, True])
 @pytest.mark.parametrize("bits", [8, 16])
-@pytest.mark.parametrize("prefix_len,tail,rows", [(64, 1, 1), (700, 3, 3), (2000, 8, 8), (129, 5, 2)])
+# Rows 3, and 5 to 8, run as groups of three, four rows as two of two: one group,
+# several, a last group of one or two rows, each over several key chunks.
+@pytest.mark.parametrize("prefix_len,tail,rows", [(64, 1, 1), (700, 3, 3), (2000, 8, 8), (129, 5, 2), (1900, 6, 4), (1500, 5, 5),
+                                                  (1030, 9, 6), (2111, 7, 7)])
 def test_decode_within_fp32_rounding_of_the_compact_oracle(fh, bits, prefix_len, tail, rows, fast):
     k, v = pair_cache(prefix_len, N_KV, 31)
     cap = prefix_len + 16

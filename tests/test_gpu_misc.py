@@ -89,9 +89,9 @@ def test_argmax_unaligned_rows_and_ties(fh):
 
 @pytest.mark.parametrize("rows,vocab", [(1, 4096), (1, 4097), (2, 65536), (3, 8195), (1, 300001), (700, 12289)])
 def test_argmax_parts(fh, rows, vocab):
-    # A row is cut into up to 64 parts of at least 4,096 logits (fewer parts
-    # with many rows): ties across the parts' borders, the ragged last part, a
-    # non-finite value in any part.
+    # A row is cut into a part for every 4,096 logits, up to 64 of them (fewer
+    # with many rows), of equal size: ties across the parts' borders, the ragged
+    # last part, a non-finite value in any part.
     parts = min(64, max(1, 1024 // rows), -(-vocab // 4096))
     chunk = -(-(-(-vocab // parts)) // 4) * 4
     logits = gen.normal((rows, vocab), 1.0, 36)
@@ -99,24 +99,30 @@ def test_argmax_parts(fh, rows, vocab):
     if rows > 1:
         logits[1, min(chunk, vocab - 1)] = logits[1, min(chunk, vocab - 1) - 1] = np.float32(9.0)
     assert fh.argmax(to_dev(logits), rows, vocab) == [int(np.argmax(r)) for r in logits]
-    logits[rows - 1, vocab - 2] = np.nan
-    with pytest.raises(fh.FocrError, match="nonfinite"):
-        fh.argmax(to_dev(logits), rows, vocab)
+    dev = to_dev(logits)
+    for at in [min(p * chunk, vocab - 1) for p in range(parts)] + [vocab - 2]:
+        kept = float(dev[rows - 1, at])
+        dev[rows - 1, at] = float("nan") if at % 2 else float("inf")
+        with pytest.raises(fh.FocrError, match="nonfinite"):
+            fh.argmax(dev, rows, vocab)
+        dev[rows - 1, at] = kept
+    assert fh.argmax(dev, rows, vocab) == [int(np.argmax(r)) for r in logits]
 
 
 def test_argmax_ties_across_partial_workgroups(fh):
-    # Rows are split into 2,048-logit partials combined per row: a tie across
-    # a partial boundary, across distant partials and inside one, a maximum in
-    # the ragged last partial, and many rows (one launch batch each 65,535).
+    # Rows of 6,149 logits are cut into two parts (3,076 logits and the rest): a
+    # tie across their border, one in each part, inside one, a maximum at the
+    # ragged end, and many rows.
     vocab = 3 * 2048 + 5
+    border = 3076
     logits = gen.normal((6, vocab), 1.0, 34)
-    logits[0, 2047] = logits[0, 2048] = np.float32(9.0)
+    logits[0, border - 1] = logits[0, border] = np.float32(9.0)
     logits[1, 6000] = logits[1, 100] = np.float32(9.0)
     logits[2, 4100] = logits[2, 4101] = np.float32(9.0)
     logits[3, vocab - 1] = np.float32(9.0)
     logits[4, :] = np.float32(0.25)
     logits[5, vocab - 5:] = np.float32(9.0)
     got = fh.argmax(to_dev(logits), 6, vocab)
-    assert got == [oracle.argmax(row) for row in logits] == [2047, 100, 4100, vocab - 1, 0, vocab - 5]
+    assert got == [oracle.argmax(row) for row in logits] == [border - 1, 100, 4100, vocab - 1, 0, vocab - 5]
     many = gen.normal((3000, 64), 1.0, 35)
     assert fh.argmax(to_dev(many), 3000, 64) == [int(np.argmax(r)) for r in many]

@@ -248,3 +248,61 @@ def test_prefill_on_the_null_stream_while_a_blocking_stream_is_captured(mode):
     assert ctx.scratch_bytes() == 0
     close(host(out).reshape(L, 16, 64), oracle.attention_prefill(q, k, v, L, L, L, 16, 8, 0, *image, sinks))
     ctx.close()
+
+
+@pytest.mark.parametrize("products", ["split", "fp32"])
+def test_captured_prefill_without_room_for_key_parts(products):
+    # 400 rows of 16 heads split their keys into parts when called eagerly; a
+    # capture with scratch for less runs them unsplit, within the same tolerance.
+    import re
+
+    import oracle
+    import torch
+
+    import focr_hip as fh
+    from test_gpu_attention import close
+
+    ctx, L, image = fh.Context(0), 400, (0, 130)
+    q, k, v = gen.normal(L * 16 * 64, 1.0, 85), gen.normal(L * 16 * 64, 1.0, 86), gen.normal(L * 8 * 64, 1.0, 87)
+    sinks = gen.uniform(16, -2.0, 2.0, 88)
+    qd, kd, vd, sd, out = (to_dev(x) for x in (q, k, v, sinks, np.zeros_like(q)))
+    kv, opts = fh.CompactKv.prefill(kd, vd, L, 16, 8), fh.PrefillOptions(split_products=products == "split")
+
+    def call():
+        fh.attention_with(qd, kv, L, fh.Geometry(0, *image), sd, opts, output=out, ctx=ctx)
+
+    def capture(expect_refusal):
+        side, g, refusal = torch.cuda.Stream(), torch.cuda.CUDAGraph(), None
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            with torch.cuda.graph(g, stream=side):
+                ctx.use_stream(torch.cuda.current_stream())
+                if expect_refusal:
+                    out.zero_()
+                    with pytest.raises(fh.FocrError, match="stream capture") as e:
+                        call()
+                    refusal = str(e.value)
+                else:
+                    call()
+        ctx.use_stream(torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        return g, refusal
+
+    if products == "split":  # the FP16 pairs of K and V need scratch of their own: reserve that and no more
+        _, refusal = capture(True)
+        ctx.reserve_scratch(int(re.search(r"grow to (\d+) bytes", refusal).group(1)))
+    sized = ctx.scratch_bytes()
+    g, _ = capture(False)
+    want = oracle.attention_prefill(q, k, v, L, L, L, 16, 8, 0, *image, sinks)
+    for rep in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        close(host(out).reshape(L, 16, 64), want)
+    assert ctx.scratch_bytes() == sized
+    call()  # eagerly the parts are taken
+    assert ctx.scratch_bytes() > sized
+    close(host(out).reshape(L, 16, 64), want)
+    del g
+    ctx.close()
