@@ -36,8 +36,6 @@ namespace focr {
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void global_void;
 
 constexpr int kQueries = 128;  // per workgroup (4 waves x 32)
 constexpr int kKeys = 32;      // per LDS key tile
@@ -106,14 +104,6 @@ __device__ __forceinline__ void copy_tile(const AttnArgs &a, KvTile &t, int ksta
     __builtin_amdgcn_global_load_lds((global_void *)(v_src),
                                      (lds_void *)(&t.rows[1][16 * j + 4 * wave][0]), 16, 0, 0);
   }
-}
-
-// Compiler-only ordering around the plain workgroup barrier: the waits are
-// explicit (a __syncthreads fence would wait for every copy in flight).
-__device__ __forceinline__ void plain_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 struct WaveState {

@@ -163,6 +163,38 @@ __device__ __forceinline__ float sdwa_cvt(uint32_t w) {
     asm("v_cvt_f32_i32_sdwa %0, sext(%1) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1" : "=v"(r) : "v"(w));
   return r;
 }
+// ---- LDS-DMA copies, barriers, tile order ------------------------------------
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) const void global_void;
+
+// s_waitcnt immediate for vmcnt(n) (n < 64) and lgkmcnt(0), expcnt not waited.
+constexpr int wait_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0070; }
+
+// Compiler-only ordering around the plain workgroup barrier: the waits are
+// explicit (a __syncthreads fence would wait for every copy in flight).
+__device__ __forceinline__ void plain_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Tile order: workgroups are dealt to the 8 XCDs round robin (block b runs on
+// XCD b % 8); block b takes tile t = (b % 8) * per + b / 8, so each XCD walks
+// a contiguous run of tiles, in panels of kTilePanel row tiles (column tiles
+// in order, rows fastest): the workgroups an XCD holds at once share a few A
+// row tiles and B column tiles in its own L2.
+constexpr int kTilePanel = 4;
+__device__ __forceinline__ void xcd_tile(int b, int row_tiles, int col_tiles, int &rt, int &ct) {
+  const int total = row_tiles * col_tiles;
+  const int per = total / 8;
+  const int t = b < 8 * per ? (b % 8) * per + b / 8 : b;
+  const int panel = t / (kTilePanel * col_tiles);
+  const int rem = t - panel * kTilePanel * col_tiles;
+  const int rows = row_tiles - panel * kTilePanel < kTilePanel ? row_tiles - panel * kTilePanel : kTilePanel;
+  ct = rem / rows;
+  rt = panel * kTilePanel + rem % rows;
+}
+
 // FP16 pairs of power-of-two scaled FP32 values (the split-product GEMM and
 // attention). A block of values (a row, a key tile, a value dim) takes the
 // exponent e of its largest finite magnitude m (2^(e-1) <= m < 2^e), and

@@ -167,34 +167,6 @@ struct GroupTile {
   float sw[BN];                // weight scales per column
 };
 
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void global_void;
-
-// Compiler-only ordering around the plain workgroup barrier: the waits are
-// explicit (a __syncthreads fence would wait for every copy in flight).
-__device__ __forceinline__ void plain_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Tile order. Workgroups are dealt to the 8 XCDs round robin (block b runs on
-// XCD b % 8); block b takes tile t = (b % 8) * per + b / 8 so that each XCD
-// walks one contiguous run of tiles, and tiles run in panels of kPanel row
-// tiles, column tiles in order, rows fastest: the workgroups an XCD holds at
-// once share a few A row tiles and B column tiles in its own L2.
-constexpr int kPanel = 4;
-__device__ __forceinline__ void tile_of(int b, int row_tiles, int col_tiles, int &rt, int &ct) {
-  const int total = row_tiles * col_tiles;
-  const int per = total / 8;
-  const int t = b < 8 * per ? (b % 8) * per + b / 8 : b;
-  const int panel = t / (kPanel * col_tiles);
-  const int rem = t - panel * kPanel * col_tiles;
-  const int rows = row_tiles - panel * kPanel < kPanel ? row_tiles - panel * kPanel : kPanel;
-  ct = rem / rows;
-  rt = panel * kPanel + rem % rows;
-}
-
 // One output: its exception FMAs (ascending columns), then the epilogue.
 // Whole waves call it (Glu exchanges neighbouring columns between lanes).
 template <int EPI>
@@ -246,7 +218,7 @@ void gemm_kernel(const int8_t *__restrict__ a_tiles, const float *__restrict__ s
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / (BN / 32), wn = wave % (BN / 32);
   int rt, ct;
-  tile_of(blockIdx.x, row_tiles, col_tiles, rt, ct);
+  xcd_tile(blockIdx.x, row_tiles, col_tiles, rt, ct);
   const int mb0 = rt * RB;
   const int nb0 = ct * (BN / 16);
   const int col_blocks = n / 16;
@@ -392,7 +364,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_small_kernel(
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int quad = lane >> 4, col_in = lane & 15;
   int rt, ct;
-  tile_of(blockIdx.x, row_tiles, col_tiles, rt, ct);
+  xcd_tile(blockIdx.x, row_tiles, col_tiles, rt, ct);
   const int mb0 = rt * RB, nb0 = (ct * WAVES + wave) * CB, col_blocks = n / 16;
   if (nb0 >= col_blocks) return;
   struct Group {

@@ -443,9 +443,6 @@ __device__ __forceinline__ float4 scale4(float4 c, float s) { return make_float4
 constexpr int kKpl = 4;  // keys per lane group per iteration (16 per wave)
 constexpr int kRoundKeys = 16 * kWaves;  // positions per workgroup round
 
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void global_void;
-
 // One workgroup per task (group g, key chunk c) serves heads 2g and 2g + 1 in
 // rounds of 64 positions: wave w takes positions 16w .. 16w + 15 of each
 // round, and the four waves' states are merged in a fixed order through LDS.
