@@ -40,7 +40,8 @@ constexpr long long kMinChunkKeys = 1024;
 // FP16-pair kernel overlap fully; those of the FP32 kernel, bound by the matrix
 // cores, hardly, and run in whole rounds. The constants are fitted to 1,790
 // measured plans of 1 to 256 heads and 9 to 16,900 visible keys: the rule loses
-// at most 4 % (FP16 pairs) and 8 % (FP32) against either plan, 0.1 % on average.
+// at most 5 % (FP16 pairs; 3 % with 16 heads) and 8 % (FP32) against either plan,
+// 0.1 % on average.
 // us per call, without / with the small parts. FP16 pairs, 16 heads, 0.6 of the
 // rows an image: 225 rows 27.5 / 25.2, 400 34.1 / 30.0, 1,000 63 / 42, 1,501 66 /
 // 55; 64 heads, 314 rows 37.0 and 37.5 (not split). FP32, 16 heads: 512 rows 47 /

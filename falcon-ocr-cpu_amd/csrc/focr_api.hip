@@ -666,8 +666,8 @@ int focr_argmax(focr_ctx *handle, const float *logits, size_t rows, size_t vocab
   if (rows == 0) return FOCR_OK;
   FOCR_REQUIRE(logits && tokens, FOCR_E_ARG, "focr_argmax: null buffer");
   FOCR_HIP_CHECK(hipSetDevice(ctx->device));
-  // Parts of at least 4,096 values (one pass of a workgroup's loads), at most
-  // 64 of them, and fewer when the rows fill the chip by themselves.
+  // A part for every 4,096 values (one pass of a workgroup's loads), all of one
+  // size, at most 64 of them, and fewer when the rows fill the chip by themselves.
   const size_t spread = std::min<size_t>(64, std::max<size_t>(1, 1024 / rows));
   const size_t parts = std::min(spread, (vocab + 4095) / 4096);
   const size_t chunk = ((vocab + parts - 1) / parts + 3) / 4 * 4;

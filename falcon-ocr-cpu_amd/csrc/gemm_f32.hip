@@ -1038,11 +1038,13 @@ union PairFrag {
 // 16 distinct bank groups. Step st reads stage st's fragments while the
 // products of stage st - 1 run. Rows and columns are padded to 128 with zeros
 // in the planes; outputs past m or n are not written.
-// Bound: the LDS and the barrier per stage beside the matrix cores. A 128-row
-// tile's stage reads 64 KB of fragments per compute unit and writes 32 KB for
-// 768 matrix-core cycles per SIMD, as many as the LDS takes; a 256-row tile's
-// takes 0.75 of that per product and has half the barriers. It holds 256
-// VGPRs (held to two waves per SIMD, a few values spilled).
+// Bound: the wait for a stage's copies and the other waves at its barrier, with
+// two waves per SIMD to cover it. W13 at 6,544 rows in 256-row tiles (counters):
+// matrix pipes busy 41 %, VALU issue 16 %, LDS active 13 %. A 256-row tile reads
+// and writes 0.75 of a 128-row tile's LDS bytes per product and meets half the
+// barriers. It holds 256 VGPRs (held to two waves per SIMD); two values (Store,
+// Add) or five (Glu) are spilled before the loop over k and reloaded after it,
+// none inside.
 template <int EPI, int BM>
 __global__ __launch_bounds__(256, BM == 256 ? 2 : 1) void split_kernel(GemmArgs a, const uint16_t *__restrict__ ap,
                                                     const uint16_t *__restrict__ bp, const int *__restrict__ aexp,

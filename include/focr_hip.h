@@ -198,7 +198,12 @@ int focr_row_scales(focr_ctx *ctx, const float *h_dev, size_t rows, size_t width
  *   prefix_len == total_len); v_dev [total_len][n_kv_heads][64];
  *   Geometry (query_offset, image_start, image_end); sinks_dev [n_heads];
  *   softmax FOCR_SOFTMAX_*; exp FOCR_EXP_*; out_dev like q.
- * FP32 matrix cores: within the FP32 tolerance of the reference tiles. */
+ * FP32 matrix cores: within the FP32 tolerance of the reference tiles.
+ * Long calls, and small ones that would leave compute units idle (from about
+ * 200 visible keys on), split their keys into parts whose states take context
+ * scratch: 540 KB a part of 16 heads. While the stream is captured and the
+ * scratch has no room for a small call's parts, the call runs unsplit: the
+ * same tolerance, another rounding than the eager call's. */
 int focr_attention_prefill(focr_ctx *ctx, const float *q_dev, const float *prefix_k_dev,
                            const float *generated_k_dev, const float *v_dev, size_t query_len,
                            size_t prefix_len, size_t total_len, size_t n_heads,
@@ -217,7 +222,8 @@ int focr_attention_prefill(focr_ctx *ctx, const float *q_dev, const float *prefi
  * holds an infinity or NaN runs focr_attention_prefill's FP32 products on the
  * device instead (its outputs bitwise that entry point's). Other geometries
  * return FOCR_E_UNSUPPORTED and write nothing (focr_attention_prefill takes
- * them). Writes K and V as FP16 pairs into the context scratch first. */
+ * them). Writes K and V as FP16 pairs into the context scratch first; splits
+ * keys as focr_attention_prefill does, by a plan of its own. */
 int focr_attention_prefill_split(focr_ctx *ctx, const float *q_dev, const float *prefix_k_dev,
                                  const float *generated_k_dev, const float *v_dev, size_t query_len,
                                  size_t prefix_len, size_t total_len, size_t n_heads,
