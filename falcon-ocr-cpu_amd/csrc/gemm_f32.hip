@@ -1390,11 +1390,13 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
   // 18.8, 32 x 64 22+.
   // The 64 x 64 form reads its operands once a wave: it gains up to one
   // workgroup per compute unit (1,024 blocks), and past that, where the launch
-  // and epilogue count for less, from a k of 2,048 on. us per call, operand
-  // planes included, 64 x 64 form / split_kernel's 64-row tiles, n = 768: 984
-  // blocks k = 192 10.9 / 11.0, 768 15.2 / 18.9, 2,304 29.0 / 43.2; 1,200 blocks
-  // k = 256 12.5 / 11.3, 768 20.3 / 18.8, 2,304 42.4 / 43.1; 2,184 blocks (2,912
-  // rows) k = 1,024 34.3 / 31.3, 2,304 59.7 / 58.7, 4,096 99.7 / 100.4.
+  // and epilogue count for less, up to two from a k of 1,024 on and further from
+  // 2,048 on. us per call, operand planes included, 64 x 64 form / split_kernel's
+  // 64-row tiles, n = 768: 984 blocks k = 192 10.9 / 11.0, 768 15.2 / 18.9, 2,304 29.0 /
+  // 43.2; 1,200 blocks k = 256 12.5 / 11.3, 768 20.3 / 18.8; 1,800 blocks k = 1,024 Store
+  // 27.6 / 26.9, Add (WO) 31.0 / 34.5; 2,184 blocks (2,912 rows) k = 1,024 34.3 / 31.3,
+  // 2,304 59.7 / 58.7, 4,096 99.7 / 100.4. One rule for all epilogues, so that Add
+  // and Glu are the Store output passed through them.
   auto launch_small = [&](auto ib, auto jb, auto wk, auto depth) {
     constexpr int IB = decltype(ib)::value, JB = decltype(jb)::value, WK = decltype(wk)::value, D = decltype(depth)::value;
     const int rt = static_cast<int>((rows + 32 * IB - 1) / (32 * IB)), ct = static_cast<int>((lin->n + 32 * JB - 1) / (32 * JB));
@@ -1411,7 +1413,7 @@ int launch_split(Ctx *ctx, const Linear *lin, const float *x, size_t rows, const
   };
   using std::integral_constant;
   const size_t blocks = ((rows + 31) / 32) * ((lin->n + 31) / 32);
-  if (blocks <= 420 || (k32 >= 192 && blocks <= 1024) || (k32 >= 2048 && blocks <= 3000)) {
+  if (blocks <= 420 || (k32 >= 192 && blocks <= 1024) || (k32 >= 1024 && blocks <= 2048) || (k32 >= 2048 && blocks <= 3000)) {
     if (blocks <= 160)
       launch_small(integral_constant<int, 1>(), integral_constant<int, 1>(), integral_constant<int, 8>(),
                    integral_constant<int, 4>());

@@ -203,11 +203,12 @@ def test_f32_split_within_fp32_tolerance(fh, m, k, n):
 
 # The small-grid forms (32 x 32, 32 x 64 and 64 x 64 outputs by the number of
 # 32 x 32 blocks): fewer k stages than a workgroup has waves, ragged edges. The
-# 64 x 64 form's lines, either side: 420 blocks at any k, 1,024 from k = 192, 3,000
-# from k = 2,048; one column tile where n has fewer columns than the planes.
+# 64 x 64 form's lines, either side: 420 blocks at any k, 1,024 from k = 192, 2,048
+# from k = 1,024, 3,000 from k = 2,048; one column tile where n has fewer columns than
+# the planes.
 @pytest.mark.parametrize("m,k,n", [(33, 40, 50), (161, 2304, 1000), (700, 300, 700), (1000, 96, 2046), (640, 190, 680),
-                                   (640, 160, 680), (1024, 192, 1022), (1030, 192, 1024), (1030, 2050, 1000), (1030, 1990, 1000),
-                                   (3000, 2048, 1000), (3010, 2048, 1022), (500, 256, 64), (5000, 256, 34)])
+                                   (640, 160, 680), (1024, 192, 1022), (1030, 192, 1024), (1030, 2050, 1000), (1030, 990, 1000),
+                                   (2040, 1024, 1020), (2050, 1024, 1020), (3000, 2048, 1000), (3010, 2048, 1022), (500, 256, 64), (5000, 256, 34)])
 def test_f32_split_small_grids(fh, m, k, n):
     test_f32_split_within_fp32_tolerance(fh, m, k, n)
 
